@@ -1121,6 +1121,9 @@ const float *oi_engine_forward(oi_engine *e, int32_t token, int32_t pos) {
 // (qwen3_5/metal.odin:22 MAX_BATCH_T; qwen3_5/engine.odin:66-93: chunks of a multiple
 // of 8 tokens, the trailing 1-7 tokens one at a time).
 constexpr int PF_MAX_T = 512;
+// K slices that every partial-product buffer has room for (a launch of several
+// projections has the slices of its tiles together, not of each projection)
+constexpr int PF_MIN_SLICES = 4;
 
 namespace {
 
@@ -1179,8 +1182,8 @@ int prefill_alloc(oi_engine *e) {
         }
         for (const auto &u : uses)
             for (int n = 8; n <= PF_MAX_T; n += 8)
-                need[u.second] = std::max(need[u.second],
-                                          (size_t)gemm_split(*u.first, n, SIZE_MAX) * n * u.first->rows * 4);
+                need[u.second] = std::max(need[u.second], (size_t)std::max(PF_MIN_SLICES, gemm_split(*u.first, n, SIZE_MAX)) *
+                                                              n * u.first->rows * 4);
     }
     need[0] = std::max(need[0], T * D * 4);  // the routed experts' weighted sums
     const size_t xb = T * std::max({D, QD, H, VD}) * 2;
@@ -1510,8 +1513,10 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
             HIP_TRY(launch_gemm_swiglu(L.w1, L.w3, e->pf_xb, T, hb, st));
             HIP_TRY(launch_gemm_parts(L.w2, hb, T, P[0], PB[0], &s0, st));
         } else {
-            HIP_TRY(launch_gemm_parts(L.w1, e->pf_xb, T, P[0], PB[0], &s0, st));
-            HIP_TRY(launch_gemm_parts(L.w3, e->pf_xb, T, P[1], PB[1], &s1, st));
+            // (OI_PREFILL_UNFUSED where the fused pass could run: unsplit as it is, the same sums)
+            const size_t one = gemm_swiglu_supported(L.w1, L.w3, T) ? (size_t)T * H * 4 : SIZE_MAX;
+            HIP_TRY(launch_gemm_parts(L.w1, e->pf_xb, T, P[0], std::min(PB[0], one), &s0, st));
+            HIP_TRY(launch_gemm_parts(L.w3, e->pf_xb, T, P[1], std::min(PB[1], one), &s1, st));
             HIP_TRY(launch_pf_swiglu16(P[0], s0, P[1], s1, (int64_t)T * H, e->pf_xb, st));
             HIP_TRY(launch_gemm_parts(L.w2, e->pf_xb, T, P[0], PB[0], &s0, st));
         }

@@ -6,29 +6,46 @@
 // X is token-major f16 [n][K], C token-major f32 [n][M] (the transposes of the
 // reference harness's B[K][N] and C[M][N]; same products).
 //
-// Work layout: a workgroup of 8 waves (two per SIMD, so that one wave's
-// dequantization overlaps the other's matrix and LDS work) computes 128 rows x
-// 64 tokens over a slice of K; wave w holds rows 16w .. 16w+15 in four
-// v_mfma_f32_16x16x32_f16 accumulators (16 tokens each).  K is walked in
-// chunks of 256 (one Q4_K / Q6_K super-block, eight Q8_0 blocks); the chunk's
-// 64 x 256 activations are staged in LDS once per workgroup and read by all
-// four waves.  Every lane dequantizes the weights it feeds to the matrix cores
-// straight from the plane layout (no LDS staging of W): lane quarter q owns one
-// 64-weight unit of the chunk (16-byte plane loads), and the chunk's eight
-// 32-wide K steps take 8 of its weights each.  The K order inside a chunk is a
-// permutation chosen so that each lane's bytes are contiguous; the activation
-// octets are placed by the same permutation (omap), so every product pairs
-// the right weight with the right activation.
+// Work layout: a workgroup of 8 waves computes 128 rows x 16 TT tokens (TT = 8,
+// 4 or 2) over a slice of K, walked in chunks of 256 (one Q4_K / Q6_K
+// super-block, eight Q8_0 blocks).  Per chunk the activations and the raw
+// weight bytes are staged in LDS; wave (rg, kh) takes rows 32 rg .. +31 and
+// half kh of the chunk's sixteen 16-wide K steps, in v_mfma_f32_32x32x16_f16
+// accumulators (TT / 2 tiles of 32 tokens), so every weight is dequantized once
+// per workgroup; the two K halves are added through LDS at the end.
+//
+// What bounds it, per chunk and CU at TT = 8 (clocks): the products 2048 (128 x
+// 128 x 256), the LDS ~2900 at 128 bytes a clock (staging, and the activations read
+// by four row groups), the vector instructions ~1900 with the products' issue,
+// the loads ~1700; alone 1.57 us a chunk, and 2.1 - 2.2 with every CU busy on
+// random data, where the card lowers its clock (a plain 8192^3 f16 product: 1795
+// TFLOP/s on zeros, 1315 on random data).  Measured on the way:
+//   - The weights go through LDS because of the loads: straight into the operand
+//     layout (16 rows x 64 bytes per instruction, the row in the fast lanes) a
+//     16-byte-per-lane load takes 65 clocks of the CU's address unit, with the
+//     four lanes of a row side by side 19-25 (L2-resident), and that alone took
+//     1560 clocks a chunk.
+//   - Two 16x16x32 products in place of one 32x32x16 hold up twice as many issue
+//     slots of the vector instructions beside them: 1.69 against 1.57 us a chunk;
+//     codes converted by v_cvt_f32_ubyte* instead of codes8: 1.84.
+//   - 128 tokens per workgroup halve the dequantization per product against 64.
+// 512 tokens, Q4_K, against 128 rows x 64 tokens with the weights loaded into the
+// operand layout: 4096 x 12288 86 -> 62 us, gate and up 2 x 12288 x 4096 with the
+// SwiGLU 159 -> 132 us; Q6_K 4096 x 12288 at 333 tokens 91.5 -> 63 us.
+//
 // Dequantization follows ggml/quant.odin exactly (separately rounded products,
 // (d*sc)*q for Q6_K), then rounds to f16 (RNE), as the reference's staging.
+// The K order inside a chunk is a permutation chosen so that each lane's bytes
+// are contiguous; the activation octets are read by the same permutation
+// (octet), so every product pairs the right weight with the right activation.
 //
 // The FFN's gate and up projections can run as one pass (gemm_q_kernel<G, 2>,
 // launch_gemm_swiglu) that writes the f16 SwiGLU of the pair instead of two
 // f32 products.
 //
-// Operand layout of v_mfma_f32_16x16x32_f16 (per lane l, 8 halves each):
-//   A[i][k]: i = l % 16, k = 8 (l / 16) + e;  B[k][j]: j = l % 16, k = 8 (l / 16) + e
-//   D[i][j] (4 floats): j = l % 16, i = 4 (l / 16) + e.
+// Operand layout of v_mfma_f32_32x32x16_f16 (per lane l, 8 halves each):
+//   A[i][k]: i = l % 32, k = 8 (l / 32) + e;  B[k][j]: j = l % 32, k = 8 (l / 32) + e
+//   D[i][j] (16 floats): j = l % 32, i = 8 (v / 4) + 4 (l / 32) + v % 4.
 
 #include <algorithm>
 
@@ -37,7 +54,10 @@
 namespace oi {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef float f32x16v __attribute__((ext_vector_type(16)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 // raw buffer descriptors (data format 32, the gfx9 value for untyped access):
@@ -50,410 +70,451 @@ static __device__ __forceinline__ u32x4 bld16(rsrc_t r, uint32_t voff, uint32_t 
     return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
 }
 
-constexpr int GM_WAVES = 8, GM_RT = 1, GM_ROWS = 16 * GM_RT * GM_WAVES, GM_TOK = 64, GM_THREADS = GM_WAVES * WAVE;
-constexpr int GM_KC = 256;                  // K per chunk
-constexpr int GM_XV = GM_TOK * GM_KC / 8;   // 16-byte activation pieces per chunk
-constexpr int GM_XPT = GM_XV / GM_THREADS;  // ... per thread
-constexpr int GM_WD = 2;                    // weight chunks in the register ring (1 in flight)
+constexpr int GM_THREADS = 512;
+constexpr int GM_ROWS = 128;  // rows per workgroup (64 of each matrix when two share it)
+constexpr int GM_KC = 256;    // K per chunk
 
-// one projection of a multi-projection launch: its matrix, partial products
-// ([split][n][rows]), K chunks per slice, row tiles, and its first block
+// one projection of a launch: its matrix, partial products ([split][n][rows]),
+// K chunks per slice, row tiles, and its first block
 struct GemmSeg {
     DMat m;
     float *c;
     int32_t cps, nx, first;
 };
 constexpr int GM_MAX_SEG = 4;
+// projections of the same x (same type and K) in one launch: a flat grid whose
+// block b belongs to the last segment with first <= b
 struct GemmArgs {
-    DMat m;             // weights [M][K], device plane layout
     const uint16_t *x;  // [n][K] f16
-    float *c;           // [n][M], or [split][n][M] partial products when K is split
-    int32_t n;
-    DMat m2;            // NP == 2: the up matrix (m is gate), same type and shape
-    uint16_t *h;        // NP == 2: [n][M] f16 silu(gate x) * (up x)
-    // nseg > 0: projections of the same x (same type and K) in one launch; a
-    // flat grid whose block b belongs to the last segment with first <= b
-    // (m, c and cps above are then unused)
-    int32_t nseg;
+    int32_t n, nseg;
     GemmSeg seg[GM_MAX_SEG];
+    DMat m2;            // two matrices: the up matrix (seg[0].m is gate), same type and shape
+    uint16_t *h;        // two matrices: [n][M] f16 silu(gate x) * (up x)
 };
 
-// f32 -> f16 (RNE) of values already rounded to f32 (f2h: the conversion is
-// kept apart from the fma that produced the value)
-static __device__ __forceinline__ h8 cvt8(const float (&v)[8]) {
-    h8 r;
+// f32 -> f16 (RNE) of values already rounded to f32 (the empty asm keeps the
+// conversion apart from the fma that produced the value, see f2h; two values
+// convert with one v_cvt_pk_f16_f32)
+static __device__ __forceinline__ h8 cvt8(float (&v)[8]) {
+    u32x4 r;
 #pragma unroll
-    for (int e = 0; e < 8; e++) r[e] = __builtin_bit_cast(_Float16, f2h(v[e]));
-    return r;
+    for (int e = 0; e < 4; e++) {
+        asm("" : "+v"(v[2 * e]));
+        asm("" : "+v"(v[2 * e + 1]));
+        r[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v{v[2 * e], v[2 * e + 1]}), h2v));
+    }
+    return __builtin_bit_cast(h8, r);
 }
 static __device__ __forceinline__ uint32_t byte_of(uint32_t lo, uint32_t hi, int e) {
     return ((e < 4 ? lo : hi) >> (8 * (e & 3))) & 0xFFu;
 }
-// keeps a masked word opaque, so that its bytes convert with v_cvt_f32_ubyte{0..3}
-// instead of being re-extracted one by one from the unmasked word
-static __device__ __forceinline__ uint32_t opaque(uint32_t v) {
-    asm volatile("" : "+v"(v));
-    return v;
+// scale q + off, rounded once to f32, of the eight codes q in the bytes of
+// (lo, hi) under mask (a code below 2^10 in each half word).  A code is
+// not converted: as f16 bits it is the denormal q 2^-24, which v_fma_mix_f32
+// takes as it is, and the scale carries the 2^24 (exactly) -- 3 instructions per
+// 4 codes where v_cvt_f32_ubyte* takes one for each after the extraction
+// (2.25 instead of 2.9 instructions per Q4_K weight in all).
+constexpr float GM_DEN = 16777216.f;  // 2^24
+static __device__ __forceinline__ void codes8(uint32_t lo, uint32_t hi, uint32_t mask, float scale, float off,
+                                              float (&v)[8]) {
+#pragma unroll
+    for (int w = 0; w < 2; w++) {
+        const uint32_t x = w ? hi : lo;
+        const h2v a = __builtin_bit_cast(h2v, x & mask), b = __builtin_bit_cast(h2v, (x >> 8) & mask);
+        v[4 * w] = __builtin_fmaf((float)a[0], scale, off);
+        v[4 * w + 1] = __builtin_fmaf((float)b[0], scale, off);
+        v[4 * w + 2] = __builtin_fmaf((float)a[1], scale, off);
+        v[4 * w + 3] = __builtin_fmaf((float)b[1], scale, off);
+    }
 }
 
-// ---- per-type raw loads and step dequantization ------------------------------
-// raw(): the bytes lane quarter q needs for chunk c of one row (issued chunks
-// ahead); deq(): the 8 weights of K step st as the A operand; omap(q, st): the
-// activation octet (8 consecutive K) those weights multiply.
+// ---- per-type staging and step dequantization ---------------------------------
+// A chunk of one row is PL planes of four 16-byte pieces (one per 64-weight unit)
+// and a 16-byte tail (scales; tail_of() the row's, one per chunk), plus for Q6_K an f16 d.
+// A lane of operand half hf owns its row's units 2 hf and 2 hf + 1: raw() takes
+// their bytes and scales for K half kh from LDS, deq(uu, i) makes the 8 weights of
+// unit 2 hf + uu, step 4 kh + i the A operand; octet(u, st): the activation octet
+// (8 consecutive K) that the weights of unit u, step st multiply.
 
-// Lane offsets: Off holds the per-lane byte offsets of one row's streams,
-// computed once; raw() adds the chunk's uniform offset.
+// one workgroup's staged weights: piece (row, q) of a plane at slot 4 row + (q ^
+// (row / 2) % 4), so 8 rows' pieces of one q fall into 8 different bank groups
+struct GmW {
+    u32x4 *pl;    // [PL][GM_THREADS]
+    u32x4 *tail;  // [GM_ROWS]
+    uint32_t *d;  // [GM_ROWS] (Q6_K)
+};
+static __device__ __forceinline__ int gm_slot(int row, int q) { return 4 * row + (q ^ ((row >> 1) & 3)); }
 
-// Q4_K, chunk = super-block c; quarter q owns unit 4c + q (bytes 0-15 in plane
-// 0, 16-31 in plane 1).  Step st = 4h + 2p + b: nibble h (group 2q + h), plane
-// p, bytes 8b .. 8b+7 of that plane; weight = 64q + 32h + 16p + 8b + e, so the
-// octet is 8q + st.  ggml/quant.odin:178-209.
+// Q4_K, chunk = super-block c; unit u of it: bytes 0-15 in plane 0, 16-31 in plane
+// 1.  Step st = 4h + 2p + b: nibble h (group 2u + h), plane p, bytes 8b .. 8b+7 of
+// that plane; weight = 64u + 32h + 16p + 8b + e, so the octet is 8u + st; K half
+// kh: nibble kh.  ggml/quant.odin:178-209.
 struct GQ4K {
-    struct Src {
-        rsrc_t q, s;
-        uint32_t plane;
-    };
-    struct Off {
-        uint32_t q, s;
-    };
+    static constexpr int PL = 2, TMAX = 8;
+    static constexpr bool D = false;
+    static __device__ __forceinline__ const u32x4 *tail_of(const DMat &m, int row) {
+        return (const u32x4 *)m.s + (size_t)row * (m.cols >> 8);
+    }
     struct Raw {
-        u32x4 p0, p1, hdr;
-    };
-    static __device__ __forceinline__ Src src(const DMat &m) {
-        return Src{make_rsrc(m.q, 2 * m.plane), make_rsrc(m.s, (size_t)m.rows * (m.cols >> 8) * 16), (uint32_t)m.plane};
-    }
-    static __device__ __forceinline__ Off off(const DMat &m, int row, int q) {
-        return Off{(uint32_t)((row * (m.cols >> 6) + q) * 16), (uint32_t)(row * (m.cols >> 8) * 16)};
-    }
-    static __device__ __forceinline__ void raw(const Src &g, const Off &o, int c, Raw &r) {
-        r.p0 = bld16(g.q, o.q, 64 * c);
-        r.p1 = bld16(g.q, o.q + g.plane, 64 * c);
-        r.hdr = bld16(g.s, o.s, 16 * c);
-    }
-    struct Pre {
+        u32x4 p[2][2];  // [unit][plane]
         float d1[2], mm[2];
     };
-    static __device__ __forceinline__ Pre pre(const Raw &r, int q) {
-        Pre p;
-        const float d = h2f(r.hdr.x & 0xFFFFu), dmin = h2f(r.hdr.x >> 16);
-        uint32_t sc0, m0, sc1, m1;
-        q4k_scales(q, r.hdr.y, r.hdr.z, r.hdr.w, sc0, m0, sc1, m1);
-        p.d1[0] = d * (float)sc0;
-        p.mm[0] = dmin * (float)m0;
-        p.d1[1] = d * (float)sc1;
-        p.mm[1] = dmin * (float)m1;
-        return p;
+    static __device__ __forceinline__ void raw(const GmW &w, int row, int hf, int kh, Raw &r) {
+        const u32x4 h = w.tail[row];
+        const float d = h2f(h.x & 0xFFFFu) * (kh ? GM_DEN / 16.f : GM_DEN), dmin = -h2f(h.x >> 16);
+#pragma unroll
+        for (int uu = 0; uu < 2; uu++) {
+            const int s = gm_slot(row, 2 * hf + uu);
+            r.p[uu][0] = w.pl[s];
+            r.p[uu][1] = w.pl[GM_THREADS + s];
+            // the unit's 24-bit field: sc(2u) | m(2u) << 6 | sc(2u+1) << 12 | m(2u+1) << 18
+            const uint32_t f = __builtin_amdgcn_alignbit(hf ? (uu ? 0u : h.w) : h.z, hf ? (uu ? h.w : h.z) : h.y,
+                                                         hf ? (uu ? 8 : 16) : (uu ? 24 : 0)) >> (12 * kh);
+            r.d1[uu] = d * (float)(f & 63u);
+            r.mm[uu] = dmin * (float)((f >> 6) & 63u);
+        }
     }
     // d1 * nib is exact in f32 (at most 11 + 6 + 4 significant bits), so the
-    // fused d1 * nib - mm rounds exactly as the separate product and difference
-    static __device__ __forceinline__ h8 deq(const Raw &r, const Pre &p, int st) {
-        const int h = st >> 2, pl = (st >> 1) & 1, b = st & 1;
-        const u32x4 &w = pl ? r.p1 : r.p0;
-        const uint32_t lo = opaque(((b ? w.z : w.x) >> (4 * h)) & 0x0F0F0F0Fu);
-        const uint32_t hi = opaque(((b ? w.w : w.y) >> (4 * h)) & 0x0F0F0F0Fu);
+    // fused d1 * nib - mm rounds exactly as the separate product and difference;
+    // the high nibbles stay where they are, 16 times their value
+    static __device__ __forceinline__ h8 deq(const Raw &r, int uu, int i, int kh) {
+        const u32x4 &w = r.p[uu][i >> 1];
         float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = __builtin_fmaf(p.d1[h], (float)byte_of(lo, hi, e), -p.mm[h]);
+        codes8((i & 1) ? w.z : w.x, (i & 1) ? w.w : w.y, kh ? 0x00F000F0u : 0x000F000Fu, r.d1[uu], r.mm[uu], v);
         return cvt8(v);
     }
-    static __device__ __forceinline__ int omap(int q, int st) { return 8 * q + st; }
+    static __device__ __forceinline__ int octet(int u, int st) { return 8 * u + st; }
 };
 
-// Q6_K, chunk = super-block c; quarter q owns unit 4c + q = unit u' = q % 2 of
-// half h = q / 2, bytes 0-15 of its ql-low, ql-high and qh planes.  Step
+// Q6_K, chunk = super-block c; unit u of it is unit u' = u % 2 of half h = u / 2,
+// bytes 0-15 of its ql-low, ql-high and qh planes.  Step
 // st = 2s + b: run s (ql-low/high nibble and qh bits 2s, scale 8h + u' + 2s),
 // bytes 8b .. 8b+7; weight = 128h + 32s + 16u' + 8b + e, octet
-// 16h + 4s + 2u' + b.  ggml/quant.odin:212-247.
+// 16h + 4s + 2u' + b.  K half kh: runs 2 kh and 2 kh + 1.  ggml/quant.odin:212-247.
 struct GQ6K {
-    struct Src {
-        rsrc_t q, s, d;
-        uint32_t plane;
-    };
-    struct Off {
-        uint32_t q, s, d;
-    };
+    static constexpr int PL = 3, TMAX = 8;
+    static constexpr bool D = true;
+    static __device__ __forceinline__ const u32x4 *tail_of(const DMat &m, int row) {
+        return (const u32x4 *)m.s + (size_t)row * (m.cols >> 8);
+    }
     struct Raw {
-        u32x4 qa, qb, qh;
-        u32x2 scw;
-        uint32_t d;
+        u32x4 l[2][2], h[2];  // [unit][ql-low, ql-high]; qh
+        float ds[2][2], off[2][2];  // [unit][run - 2 kh]
     };
-    static __device__ __forceinline__ Src src(const DMat &m) {
-        const size_t nsb = (size_t)m.rows * (m.cols >> 8);
-        return Src{make_rsrc(m.q, 3 * m.plane), make_rsrc(m.s, nsb * 16), make_rsrc(m.d, nsb * 2), (uint32_t)m.plane};
-    }
-    static __device__ __forceinline__ Off off(const DMat &m, int row, int q) {
-        const int nsb = m.cols >> 8;
-        return Off{(uint32_t)((row * (m.cols >> 6) + q) * 16), (uint32_t)(row * nsb * 16 + 8 * (q >> 1)),
-                   (uint32_t)(row * nsb * 2)};
-    }
-    static __device__ __forceinline__ void raw(const Src &g, const Off &o, int c, Raw &r) {
-        r.qa = bld16(g.q, o.q, 64 * c);
-        r.qb = bld16(g.q, o.q + g.plane, 64 * c);
-        r.qh = bld16(g.q, o.q + 2 * g.plane, 64 * c);
-        r.scw = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(g.s, o.s, 16 * c, 0));
-        r.d = __builtin_amdgcn_raw_buffer_load_b16(g.d, o.d, 2 * c, 0);
-    }
-    struct Pre {
-        float ds[4], off[4];
-    };
-    static __device__ __forceinline__ Pre pre(const Raw &r, int q) {
-        Pre p;
-        const float d = h2f(r.d);
+    static __device__ __forceinline__ void raw(const GmW &w, int row, int hf, int kh, Raw &r) {
+        // unit 2 hf + u' is unit u' of half hf; scales 8 hf + u' + 2s of runs s = 2 kh,
+        // 2 kh + 1: bytes u' and u' + 2 of one word
+        const uint32_t sw = ((const uint32_t *)(w.tail + row))[2 * hf + kh];
+        const float d = h2f(w.d[row]);
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int is = (q & 1) + 2 * s;
-            p.ds[s] = d * (float)(int8_t)byte_of(r.scw.x, r.scw.y, is);
-            p.off[s] = -32.f * p.ds[s];
+        for (int uu = 0; uu < 2; uu++) {
+            const int s = gm_slot(row, 2 * hf + uu);
+            r.l[uu][0] = w.pl[s];
+            r.l[uu][1] = w.pl[GM_THREADS + s];
+            r.h[uu] = w.pl[2 * GM_THREADS + s];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float ds = d * (float)(int8_t)((sw >> (8 * uu + 16 * j)) & 0xFFu);
+                r.ds[uu][j] = ds * GM_DEN;
+                r.off[uu][j] = -32.f * ds;
+            }
         }
-        return p;
     }
     // ds * (code - 32) as one fused ds * code - 32 ds: the exact value is the
     // same and the fma rounds it once, as the reference's single product
-    static __device__ __forceinline__ h8 deq(const Raw &r, const Pre &p, int st) {
-        const int s = st >> 1, b = st & 1;
-        const u32x4 &l = (s & 1) ? r.qb : r.qa;
-        const uint32_t llo = ((b ? l.z : l.x) >> (4 * (s >> 1))) & 0x0F0F0F0Fu;
-        const uint32_t lhi = ((b ? l.w : l.y) >> (4 * (s >> 1))) & 0x0F0F0F0Fu;
-        const uint32_t hlo = (((b ? r.qh.z : r.qh.x) >> (2 * s)) & 0x03030303u) << 4;
-        const uint32_t hhi = (((b ? r.qh.w : r.qh.y) >> (2 * s)) & 0x03030303u) << 4;
-        const uint32_t wlo = opaque(llo | hlo), whi = opaque(lhi | hhi);  // 6-bit codes, one per byte
+    static __device__ __forceinline__ h8 deq(const Raw &r, int uu, int i, int kh) {
+        const int j = i >> 1, b = i & 1;
+        const u32x4 &l = r.l[uu][j], &h = r.h[uu];
+        const uint32_t llo = ((b ? l.z : l.x) >> (4 * kh)) & 0x0F0F0F0Fu;
+        const uint32_t lhi = ((b ? l.w : l.y) >> (4 * kh)) & 0x0F0F0F0Fu;
+        const uint32_t hlo = (((b ? h.z : h.x) >> (4 * kh + 2 * j)) & 0x03030303u) << 4;
+        const uint32_t hhi = (((b ? h.w : h.y) >> (4 * kh + 2 * j)) & 0x03030303u) << 4;
         float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = __builtin_fmaf(p.ds[s], (float)byte_of(wlo, whi, e), p.off[s]);
+        codes8(llo | hlo, lhi | hhi, 0x00FF00FFu, r.ds[uu][j], r.off[uu][j], v);  // 6-bit codes, one per byte
         return cvt8(v);
     }
-    static __device__ __forceinline__ int omap(int q, int st) {
-        return 16 * (q >> 1) + 4 * (st >> 1) + 2 * (q & 1) + (st & 1);
+    static __device__ __forceinline__ int octet(int u, int st) {
+        return 16 * (u >> 1) + 4 * (st >> 1) + 2 * (u & 1) + (st & 1);
     }
 };
 
-// Q8_0, chunk = blocks 8c .. 8c+7; quarter q owns unit 4c + q (blocks 8c + 2q
-// and 8c + 2q + 1); plane 2 blk + half holds bytes 16 half .. +15 of block blk.
-// Step st = 4 blk + 2 half + b: weight 64q + 8st + e, octet 8q + st.
-// ggml/quant.odin:87-96.
+// Q8_0, chunk = blocks 8c .. 8c+7; unit u of it: blocks 8c + 2u and 8c + 2u + 1;
+// plane 2 blk + half holds bytes 16 half .. +15 of block blk.  Step st = 4 blk + 2
+// half + b: weight 64u + 8st + e, octet 8u + st; K half kh: block kh of the unit.  (Four planes beside 128 tokens would not fit the LDS:
+// TMAX 4.)  ggml/quant.odin:87-96.
 struct GQ80 {
-    struct Src {
-        rsrc_t q, d;
-        uint32_t plane;
-    };
-    struct Off {
-        uint32_t q, d;
-    };
+    static constexpr int PL = 4, TMAX = 4;
+    static constexpr bool D = false;
+    static __device__ __forceinline__ const u32x4 *tail_of(const DMat &m, int row) {  // eight block scales per chunk
+        return (const u32x4 *)m.d + (size_t)row * (m.cols >> 8);
+    }
     struct Raw {
-        u32x4 pl[4];
-        uint32_t d;
-    };
-    static __device__ __forceinline__ Src src(const DMat &m) {
-        return Src{make_rsrc(m.q, 4 * m.plane), make_rsrc(m.d, (size_t)m.rows * (m.cols >> 5) * 2), (uint32_t)m.plane};
-    }
-    static __device__ __forceinline__ Off off(const DMat &m, int row, int q) {
-        return Off{(uint32_t)((row * (m.cols >> 6) + q) * 16), (uint32_t)((row * (m.cols >> 5) + 2 * q) * 2)};
-    }
-    static __device__ __forceinline__ void raw(const Src &g, const Off &o, int c, Raw &r) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) r.pl[k] = bld16(g.q, o.q + k * g.plane, 64 * c);
-        r.d = __builtin_amdgcn_raw_buffer_load_b32(g.d, o.d, 16 * c, 0);
-    }
-    struct Pre {
+        u32x4 p[2][2];  // [unit][half of block kh]
         float d[2];
     };
-    static __device__ __forceinline__ Pre pre(const Raw &r, int) {
-        return Pre{{h2f(r.d & 0xFFFFu), h2f(r.d >> 16)}};
+    static __device__ __forceinline__ void raw(const GmW &w, int row, int hf, int kh, Raw &r) {
+#pragma unroll
+        for (int uu = 0; uu < 2; uu++) {
+            const int s = gm_slot(row, 2 * hf + uu);
+            r.p[uu][0] = w.pl[2 * kh * GM_THREADS + s];
+            r.p[uu][1] = w.pl[(2 * kh + 1) * GM_THREADS + s];
+            r.d[uu] = h2f((((const uint32_t *)(w.tail + row))[2 * hf + uu] >> (16 * kh)) & 0xFFFFu);
+        }
     }
-    static __device__ __forceinline__ h8 deq(const Raw &r, const Pre &p, int st) {
+    static __device__ __forceinline__ h8 deq(const Raw &r, int uu, int i, int) {
 #pragma clang fp contract(off)
-        const u32x4 &w = r.pl[st >> 1];
-        const int b = st & 1;
-        const uint32_t lo = b ? w.z : w.x, hi = b ? w.w : w.y;
+        const u32x4 &w = r.p[uu][i >> 1];
+        const uint32_t lo = (i & 1) ? w.z : w.x, hi = (i & 1) ? w.w : w.y;
         float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = p.d[st >> 2] * (float)(int8_t)byte_of(lo, hi, e);
+        for (int e = 0; e < 8; e++) v[e] = r.d[uu] * (float)(int8_t)byte_of(lo, hi, e);
         return cvt8(v);
     }
-    static __device__ __forceinline__ int omap(int q, int st) { return 8 * q + st; }
+    static __device__ __forceinline__ int octet(int u, int st) { return 8 * u + st; }
 };
 
-// One workgroup: rows [128 bx, +128), tokens [64 by, +64), chunks
-// [bz * cps, +cps) of K.  Activations: chunk c + 1 is loaded into registers
-// while chunk c is computed, then stored to the LDS buffer of its parity
-// (piece (token j, octet o) at slot 64 o + (j ^ (o % 8)): conflict-free stores
-// of 8 consecutive octets and conflict-free 16-lane operand reads); weights
-// run GM_WD - 1 chunks ahead in a register ring.  With more than one K slice
-// (split > 1) slice z writes its partial products to c + z n M; gemm_reduce
-// sums them in slice order.
+template <class G>
+static constexpr size_t gm_lds(int tt) {
+    return (size_t)2 * 16 * tt * (GM_KC / 8) * 16 + (size_t)G::PL * GM_THREADS * 16 + GM_ROWS * 16 + (G::D ? GM_ROWS * 4 : 0);
+}
+
+// One workgroup: 128 rows (NP == 2: 64 rows of each matrix), 16 TT tokens, a
+// slice of cps chunks of K.  Chunk c + 1 is loaded into registers while chunk c
+// is computed and stored to LDS when chunk c's weights have been taken out of
+// it: activations double-buffered (piece (token j, octet o) at slot TOK o + (j ^
+// (o % 8)): conflict-free stores of 8 consecutive octets and conflict-free
+// 16-lane operand reads), weights in one buffer that every wave copies its
+// operand bytes from first.  With more than one K slice (split > 1) slice z
+// writes its partial products to c + z n M; the consumer sums them in slice
+// order.
 //
-// NP == 2 (gate and up of the FFN, one K slice): both matrices' rows are
-// computed against the same staged activations, each B operand read from LDS
-// feeding both products, and the epilogue writes the f16 SwiGLU of the pair
-// (infer/forward.odin:128-132: v *= 1/(1+exp(-v)); v *= up; then the half
-// staging of the next projection's input).
-template <class G, int NP = 1>
-__global__ __launch_bounds__(GM_THREADS) void gemm_q_kernel(GemmArgs a, int cps) {
-    __shared__ __attribute__((aligned(16))) u32x4 xs[2][GM_XV];
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-    const int q = lane >> 4, li = lane & 15;
-    // the block's matrix, output and (row tile, token tile, K slice)
-    DMat mat = a.m;
-    float *cout = a.c;
-    int bx = (int)blockIdx.x, by = (int)blockIdx.y, bz = (int)blockIdx.z;
-    if (NP == 1 && a.nseg > 0) {
-        int sg = 0;
-#pragma unroll
-        for (int i = 1; i < GM_MAX_SEG; i++)
-            if (i < a.nseg && bx >= a.seg[i].first) sg = i;
-        const GemmSeg &g = a.seg[sg];
-        const int ny = (a.n + GM_TOK - 1) / GM_TOK, loc = bx - g.first;
-        mat = g.m;
-        cout = g.c;
-        cps = g.cps;
-        bz = loc / (g.nx * ny);
-        by = (loc - bz * g.nx * ny) / g.nx;
-        bx = loc - bz * g.nx * ny - by * g.nx;
+// NP == 2 (gate and up of the FFN, one K slice): the operand's rows 0-15 are the
+// gate matrix's, 16-31 the up matrix's same rows, and the epilogue writes the f16
+// SwiGLU of the pair (infer/forward.odin:128-132: v *= 1/(1+exp(-v)); v *= up;
+// then the half staging of the next projection's input).
+//
+// Consecutive blocks go to different XCDs; the block index is turned so that
+// each XCD takes a contiguous range of (slice, row tile, token tile), the token
+// tiles of one row tile together: its L2 reads those weights once.
+template <class G, int NP, int TT>
+__global__ __launch_bounds__(GM_THREADS) void gemm_q_kernel(GemmArgs a) {
+    constexpr int TOK = 16 * TT, TH = TT / 2, XV = TOK * GM_KC / 8, XPT = XV / GM_THREADS, PL = G::PL;
+    extern __shared__ __attribute__((aligned(16))) u32x4 gm_smem[];
+    u32x4 *xs = gm_smem;  // [2][XV]
+    GmW ws;
+    ws.pl = gm_smem + 2 * XV;
+    ws.tail = ws.pl + PL * GM_THREADS;
+    ws.d = (uint32_t *)(ws.tail + GM_ROWS);
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), hf = lane >> 5, li = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), rg = wave >> 1, kh = wave & 1;
+    // the block's projection, row tile, token tile and K slice
+    int b = (int)blockIdx.x;
+    {
+        const int nb = (int)gridDim.x, per = nb >> 3, rem = nb & 7, xcd = b & 7;
+        b = xcd * per + min(xcd, rem) + (b >> 3);
     }
-    const int M = mat.rows, K = mat.cols;
-    const int rbase = bx * GM_ROWS + 16 * GM_RT * wave;
-    typename G::Src src[NP];
-    src[0] = G::src(mat);
-    if (NP == 2) src[NP - 1] = G::src(a.m2);  // same shape: the same lane offsets
-    typename G::Off off[GM_RT];
+    int sg = 0;
 #pragma unroll
-    for (int rt = 0; rt < GM_RT; rt++) off[rt] = G::off(mat, min(rbase + 16 * rt + li, M - 1), q);  // rows past M: not stored
-    const int t0 = by * GM_TOK;
-    const int nchunk = K / GM_KC;
-    const int c0 = bz * cps, c1 = min(nchunk, c0 + cps);
+    for (int i = 1; i < GM_MAX_SEG; i++)
+        if (i < a.nseg && b >= a.seg[i].first) sg = i;
+    const GemmSeg &g = a.seg[sg];
+    const DMat &mat = g.m;
+    const int ny = (a.n + TOK - 1) / TOK, loc = b - g.first, bz = loc / (g.nx * ny);
+    const int bx = (loc - bz * g.nx * ny) / ny, t0 = (loc - (bz * g.nx + bx) * ny) * TOK;
+    const int M = mat.rows, K = mat.cols, nchunk = K / GM_KC;
+    const int c0 = bz * g.cps, c1 = min(nchunk, c0 + g.cps);
 
+    // local row lr = 32 rg + i: matrix row (rows past M: read, not stored)
+    auto row_of = [&](int lr) {
+        return min(NP == 2 ? bx * (GM_ROWS / 2) + (lr >> 5) * 16 + (lr & 15) : bx * GM_ROWS + lr, M - 1);
+    };
+    // staging loads: piece tid % 4 of local row tid / 4 per plane, the tail of row tid
+    const size_t pbytes = (size_t)PL * mat.plane;
+    // (two matrices: the wave's pieces are of one of them)
+    const bool tsecond = NP == 2 && (tid & 16);
+    const uint32_t woff = (uint32_t)((row_of(tid >> 2) * (K >> 6) + (tid & 3)) * 16);
+    const int trow = row_of(tid & (GM_ROWS - 1));
+    const rsrc_t wsrc = make_rsrc(NP == 2 && (wave & 1) ? a.m2.q : mat.q, pbytes);
+    const u32x4 *tsrc = G::tail_of(tsecond ? a.m2 : mat, trow);
+    const uint16_t *dsrc = (tsecond ? a.m2.d : mat.d) + (size_t)trow * (K >> 8);
     const rsrc_t xsrc = make_rsrc(a.x, (size_t)a.n * K * 2);
-    uint32_t xoff[GM_XPT];
+    uint32_t xoff[XPT];
 #pragma unroll
-    for (int i = 0; i < GM_XPT; i++) {
-        const int p = threadIdx.x + i * GM_THREADS, j = p >> 5, o = p & 31;
-        xoff[i] = (uint32_t)(min(t0 + j, a.n - 1) * K * 2 + 16 * o);
+    for (int i = 0; i < XPT; i++) {
+        const int p = tid + i * GM_THREADS;
+        xoff[i] = (uint32_t)(min(t0 + (p >> 5), a.n - 1) * K * 2 + 16 * (p & 31));
     }
-    u32x4 xr[GM_XPT];
-    auto xfetch = [&](int c) {
-#pragma unroll
-        for (int i = 0; i < GM_XPT; i++) xr[i] = bld16(xsrc, xoff[i], c * GM_KC * 2);
+    // a chunk on its way from memory to LDS, in registers
+    struct Stage {
+        u32x4 x[XPT], w[PL], t;
+        uint32_t d;
     };
-    auto xstore = [&](int buf) {
+    auto wfetch = [&](int c, Stage &r) {
 #pragma unroll
-        for (int i = 0; i < GM_XPT; i++) {
-            const int p = threadIdx.x + i * GM_THREADS, j = p >> 5, o = p & 31;
-            xs[buf][o * GM_TOK + (j ^ (o & 7))] = xr[i];
+        for (int k = 0; k < PL; k++) r.w[k] = bld16(wsrc, woff + (uint32_t)(k * mat.plane), 64 * c);
+        if (tid < GM_ROWS) {
+            r.t = tsrc[c];
+            if constexpr (G::D) r.d = dsrc[c];
         }
     };
+    auto wstore = [&](const Stage &r) {
+#pragma unroll
+        for (int k = 0; k < PL; k++) ws.pl[k * GM_THREADS + gm_slot(tid >> 2, tid & 3)] = r.w[k];
+        if (tid < GM_ROWS) {
+            ws.tail[tid] = r.t;
+            if constexpr (G::D) ws.d[tid] = r.d;
+        }
+    };
+    auto xfetch = [&](int c, int i, Stage &r) { r.x[i] = bld16(xsrc, xoff[i], c * GM_KC * 2); };
+    u32x4 *const xput = xs + (tid & 31) * TOK + ((tid >> 5) ^ (tid & 7));  // piece tid's slot; piece tid + 512 i's: 16 i on
+    auto xstore = [&](int buf, int i, const Stage &r) { xput[buf * XV + 16 * i] = r.x[i]; };
+    Stage next;
 
-    f32x4v acc[NP][GM_RT][4];
+    f32x16v acc[TH];
 #pragma unroll
-    for (int mp = 0; mp < NP; mp++)
+    for (int t = 0; t < TH; t++)
 #pragma unroll
-        for (int rt = 0; rt < GM_RT; rt++)
+        for (int e = 0; e < 16; e++) acc[t][e] = 0.f;
+    // Software pipeline over the K half's eight 16-wide K steps: a step's products
+    // run beside the next step's operand reads and dequantization and a part of the
+    // next chunk's staging (issued together ahead of the products, the staging
+    // alone held the waves up for longer than the products take).  Barrier Q (step
+    // 2): every wave has taken chunk c's weights out of LDS and is done with chunk
+    // c - 1's activations, so chunk c + 1 may be stored over them.  Barrier P
+    // (step 6): chunk c + 1 is staged; steps 6 and 7 read ahead into it.
+    constexpr int XQ = (XPT + 3) / 4;  // X pieces staged in each of steps 2 - 5
+    typename G::Raw raw;
+    h8 A[2], B[2][TH];
+    auto readx = [&](int buf, int s, h8 (&d)[TH]) {
+        const int o = G::octet(2 * hf + (s >> 2), 4 * kh + (s & 3));
+        const u32x4 *xp = xs + buf * XV + o * TOK + (li ^ (o & 7));
 #pragma unroll
-            for (int t = 0; t < 4; t++) acc[mp][rt][t] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    // unconditional loads: chunks past the slice re-read its first, unused
-    typename G::Raw ring[GM_WD][NP][GM_RT];
+        for (int t = 0; t < TH; t++) d[t] = __builtin_bit_cast(h8, xp[32 * t]);
+    };
+    if (c0 < c1) {
+        // the first two chunks are requested together (the second after the first
+        // had arrived, every workgroup waited for memory twice)
+        Stage first;
+        const int cs = min(c0 + 1, c1 - 1);
+        wfetch(c0, first);
 #pragma unroll
-    for (int r = 0; r < GM_WD - 1; r++)
+        for (int i = 0; i < XPT; i++) xfetch(c0, i, first);
+        wfetch(cs, next);
 #pragma unroll
-        for (int mp = 0; mp < NP; mp++)
+        for (int i = 0; i < XPT; i++) xfetch(cs, i, next);
+        wstore(first);
 #pragma unroll
-            for (int rt = 0; rt < GM_RT; rt++)
-                G::raw(src[mp], off[rt], c0 + r < c1 ? c0 + r : c0, ring[r][mp][rt]);
-    if (c0 < c1) xfetch(c0);
-    for (int cb = c0; cb < c1; cb += GM_WD) {
+        for (int i = 0; i < XPT; i++) xstore(0, i, first);
+        __syncthreads();
+        G::raw(ws, 32 * rg + li, hf, kh, raw);
+        readx(0, 0, B[0]);
+        A[0] = G::deq(raw, 0, 0, kh);
+    }
+    for (int c = c0; c < c1; c++) {
+        const int buf = (c - c0) & 1, cn = min(c + 2, c1 - 1);
 #pragma unroll
-        for (int r = 0; r < GM_WD; r++) {
-            const int c = cb + r;
-            if (c >= c1) break;
-            const int cn = c + GM_WD - 1 < c1 ? c + GM_WD - 1 : c0;
-#pragma unroll
-            for (int mp = 0; mp < NP; mp++)
-#pragma unroll
-                for (int rt = 0; rt < GM_RT; rt++) G::raw(src[mp], off[rt], cn, ring[(r + GM_WD - 1) % GM_WD][mp][rt]);
-            const int buf = (c - c0) & 1;
-            xstore(buf);
-            if (c + 1 < c1) xfetch(c + 1);
-            __syncthreads();  // chunk c staged; every wave is done with chunk c - 2's buffer
-            typename G::Pre pre[NP][GM_RT];
-#pragma unroll
-            for (int mp = 0; mp < NP; mp++)
-#pragma unroll
-                for (int rt = 0; rt < GM_RT; rt++) pre[mp][rt] = G::pre(ring[r][mp][rt], q);
-#pragma unroll
-            for (int st = 0; st < 8; st++) {
-                const int o = G::omap(q, st);
-                h8 B[4];
-#pragma unroll
-                for (int t = 0; t < 4; t++) B[t] = __builtin_bit_cast(h8, xs[buf][o * GM_TOK + ((16 * t + li) ^ (o & 7))]);
-#pragma unroll
-                for (int mp = 0; mp < NP; mp++)
-#pragma unroll
-                    for (int rt = 0; rt < GM_RT; rt++) {
-                        const h8 A = G::deq(ring[r][mp][rt], pre[mp][rt], st);
-#pragma unroll
-                        for (int t = 0; t < 4; t++)
-                            acc[mp][rt][t] =
-                                __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[t], acc[mp][rt][t], 0, 0, 0);
-                    }
+        for (int s = 0; s < 8; s++) {
+            const int cur = s & 1, nxt = cur ^ 1, sn = (s + 1) & 7;
+            if (s == 2) {
+                __syncthreads();  // Q
+                wstore(next);
+                wfetch(cn, next);
             }
+            if (s == 6) __syncthreads();  // P
+            if (s == 7) G::raw(ws, 32 * rg + li, hf, kh, raw);  // (past the last chunk: that chunk again, unused)
+            readx(s == 7 ? buf ^ 1 : buf, sn, B[nxt]);
+            if (s >= 2 && s < 6) {
+#pragma unroll
+                for (int j = XQ * (s - 2); j < XQ * (s - 1) && j < XPT; j++) {
+                    xstore(buf ^ 1, j, next);
+                    xfetch(cn, j, next);
+                }
+            }
+            A[nxt] = G::deq(raw, sn >> 2, sn & 3, kh);
+#pragma unroll
+            for (int t = 0; t < TH; t++)
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[cur], B[cur][t], acc[t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // D of tile (rt, t): lane (j, g) holds rows 4g .. 4g+3 of column (token) j
-    if (NP == 2) {
+    // the two K halves through LDS ([kh][token][row], the row's 16-byte pieces
+    // turned by the token against bank conflicts), then coalesced stores of
+    // their sums: lane (j, h) of tile t holds rows 8 g + 4 h .. +3 of token j in
+    // floats 4 g .. 4 g + 3
+    __syncthreads();
+    f32x4v *yo = (f32x4v *)gm_smem;  // [2][TOK][32]
 #pragma unroll
-        for (int rt = 0; rt < GM_RT; rt++) {
-            const int r0 = rbase + 16 * rt + 4 * q;
+    for (int t = 0; t < TH; t++)
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int tk = t0 + 16 * t + li;
-                if (tk >= a.n) continue;
-                uint16_t hv[4];
+        for (int g = 0; g < 4; g++) {
+            const int tk = 32 * t + li;
+            yo[(kh * TOK + tk) * 32 + ((8 * rg + 2 * g + hf) ^ (tk & 7))] =
+                f32x4v{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+        }
+    __syncthreads();
+    auto sum = [&](int tk, int col) {
+        const int i = tk * 32 + (col ^ (tk & 7));
+        return yo[i] + yo[TOK * 32 + i];
+    };
+    if constexpr (NP == 2) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
+        for (int i = 0; i < TOK * 16 / GM_THREADS; i++) {
+            const int p = tid + i * GM_THREADS, tk = p >> 4, cc = p & 15;  // row piece 4 cc of the 64 rows
+            if (t0 + tk >= a.n) continue;
+            const f32x4v gv = sum(tk, 8 * (cc >> 2) + (cc & 3)), uv = sum(tk, 8 * (cc >> 2) + 4 + (cc & 3));
+            uint16_t hv[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
 #pragma clang fp contract(off)
-                    float v = acc[0][rt][t][e];
-                    v *= 1.0f / (1.0f + expf(-v));
-                    v *= acc[NP - 1][rt][t][e];
-                    hv[e] = f2h(v);
-                }
-                uint16_t *dst = a.h + (size_t)tk * M + r0;
-                if (r0 + 3 < M && (M & 3) == 0) {
-                    *(u32x2 *)dst = u32x2{(uint32_t)hv[0] | ((uint32_t)hv[1] << 16),
-                                          (uint32_t)hv[2] | ((uint32_t)hv[3] << 16)};
-                    continue;
-                }
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (r0 + e < M) dst[e] = hv[e];
+                float v = gv[e];
+                v *= 1.0f / (1.0f + expf(-v));
+                v *= uv[e];
+                hv[e] = f2h(v);
             }
-        }
-        return;
-    }
-    float *out = cout + (size_t)bz * a.n * M;
-#pragma unroll
-    for (int rt = 0; rt < GM_RT; rt++) {
-        const int r0 = rbase + 16 * rt + 4 * q;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int tk = t0 + 16 * t + li;
-            if (tk >= a.n) continue;
-            float *dst = out + (size_t)tk * M + r0;
+            const int r0 = bx * (GM_ROWS / 2) + 4 * cc;
+            uint16_t *dst = a.h + (size_t)(t0 + tk) * M + r0;
             if (r0 + 3 < M && (M & 3) == 0) {
-                *(f32x4v *)dst = acc[0][rt][t];
+                *(u32x2 *)dst = u32x2{(uint32_t)hv[0] | ((uint32_t)hv[1] << 16), (uint32_t)hv[2] | ((uint32_t)hv[3] << 16)};
                 continue;
             }
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if (r0 + e < M) dst[e] = acc[0][rt][t][e];
+                if (r0 + e < M) dst[e] = hv[e];
+        }
+    } else {
+        float *out = g.c + (size_t)bz * a.n * M;
+#pragma unroll
+        for (int i = 0; i < XPT; i++) {
+            const int p = tid + i * GM_THREADS, tk = p >> 5, cc = p & 31;
+            if (t0 + tk >= a.n) continue;
+            const f32x4v v = sum(tk, cc);
+            const int r0 = bx * GM_ROWS + 4 * cc;
+            float *dst = out + (size_t)(t0 + tk) * M + r0;
+            if (r0 + 3 < M && (M & 3) == 0) {
+                *(f32x4v *)dst = v;
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (r0 + e < M) dst[e] = v[e];
         }
     }
 }
 
-// c[i] = sum over slices z (in order) of part[z][i]
+// c[i] = sum over slices z (in order) of part[z][i]; eight slices' loads are in
+// flight together (a loop of load and add waits for each in turn)
 __global__ __launch_bounds__(WG) void gemm_reduce(const float *part, float *c, int64_t total, int split) {
     const int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x;
     if (4 * i + 3 < total) {
-        f32x4v s = *(const f32x4v *)(part + 4 * i);
-        for (int z = 1; z < split; z++) s += *(const f32x4v *)(part + z * total + 4 * i);
+        f32x4v s = {0.f, 0.f, 0.f, 0.f};
+        for (int z0 = 0; z0 < split; z0 += 8) {
+            f32x4v v[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = *(const f32x4v *)(part + min(z0 + k, split - 1) * total + 4 * i);
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+                if (z0 + k < split) s = z0 + k ? s + v[k] : v[k];
+        }
         *(f32x4v *)(c + 4 * i) = s;
     } else {
         for (int64_t k = 4 * i; k < total; k++) {
@@ -473,16 +534,70 @@ static int normalize_split(int nchunk, int split) {
     return (nchunk + cps - 1) / cps;
 }
 
-// K is split so that about 256 workgroups run (one per CU; each slice at least
-// two chunks; measured best on 4096/12288 x 64 x 4096/12288), and no further
-// than the partial-product buffer holds.
-int gemm_split(const DMat &m, int32_t n, size_t part_bytes) {
-    const int nchunk = m.cols / GM_KC;
-    const int tiles = ((m.rows + GM_ROWS - 1) / GM_ROWS) * ((n + GM_TOK - 1) / GM_TOK);
-    int split = std::max(1, std::min((256 + tiles / 2) / tiles, nchunk / 2));
-    const size_t per = (size_t)n * m.rows * 4;
-    split = (int)std::min<size_t>(split, std::max<size_t>(1, part_bytes / per));
-    return normalize_split(nchunk, split);
+// Token tiles (of 16) per workgroup and K split of a launch of `rt` row tiles: the
+// pair of least estimated time with at most `cap` slices.  Estimated (us, measured
+// on 4096 x n x 4096 / 12288 with every CU busy): a chunk at 128 tokens 2.2, 64
+// tokens 1.6, 32 tokens 0.9; a workgroup's fixed time; rounds of one workgroup per
+// CU; the further slices written and read back; the reduction's launch if the
+// caller has one.
+struct GemmPlan {
+    int tt, split;
+};
+static GemmPlan gemm_plan(int type, int rt, int nchunk, int32_t n, double out, int cap, bool reduce) {
+    GemmPlan best{0, 1};
+    double bt = 1e30;
+    const int tmax = n <= 32 ? 2 : n <= 64 || type == T_Q8_0 ? 4 : 8;
+    for (int tt = n <= 32 ? 2 : 4; tt <= tmax; tt *= 2) {
+        const double chunk = tt == 8 ? 2.2 : tt == 4 ? 1.6 : 0.9, fixed = tt == 8 ? 5.0 : 4.0;
+        const int tiles = rt * ((n + 16 * tt - 1) / (16 * tt));
+        for (int s = 1; s <= std::max(1, nchunk / 2) && s <= cap; s++) {
+            if (normalize_split(nchunk, s) != s) continue;
+            const double t = (tiles * s + 255) / 256 * (((nchunk + s - 1) / s) * chunk + fixed) +
+                             (s > 1 ? (s - 1) * out * 8.0 / 8e6 + (reduce ? 4.0 : 0.0) : 0.0);
+            if (t < bt) {
+                bt = t;
+                best = GemmPlan{tt, s};
+            }
+        }
+    }
+    return best;
+}
+static int gemm_rt(const DMat &m, int rows = GM_ROWS) { return (m.rows + rows - 1) / rows; }
+static int gemm_cap(const DMat &m, int32_t n, size_t part_bytes) {
+    return (int)std::max<size_t>(1, std::min<size_t>(64, part_bytes / ((size_t)n * m.rows * 4)));
+}
+static GemmPlan gemm_plan(const DMat &m, int32_t n, size_t part_bytes) {
+    return gemm_plan(m.type, gemm_rt(m), m.cols / GM_KC, n, (double)n * m.rows, gemm_cap(m, n, part_bytes), true);
+}
+
+int gemm_split(const DMat &m, int32_t n, size_t part_bytes) { return gemm_plan(m, n, part_bytes).split; }
+
+template <class G, int NP>
+static hipError_t gemm_launch_t(const GemmArgs &a, int blocks, int tt, hipStream_t st) {
+    const dim3 grid((unsigned)blocks), block(GM_THREADS);
+    switch (tt) {
+    case 2: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 2>), grid, block, gm_lds<G>(2), st, a); break;
+    case 4: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 4>), grid, block, gm_lds<G>(4), st, a); break;
+    default:
+        if constexpr (G::TMAX >= 8) hipLaunchKernelGGL((gemm_q_kernel<G, NP, 8>), grid, block, gm_lds<G>(8), st, a);
+        else return hipErrorInvalidValue;
+        break;
+    }
+    return hipGetLastError();
+}
+template <int NP>
+static hipError_t gemm_launch(const GemmArgs &a, int blocks, int tt, hipStream_t st) {
+    switch (a.seg[0].m.type) {
+    case T_Q4_K: return gemm_launch_t<GQ4K, NP>(a, blocks, tt, st);
+    case T_Q6_K: return gemm_launch_t<GQ6K, NP>(a, blocks, tt, st);
+    default: return gemm_launch_t<GQ80, NP>(a, blocks, tt, st);
+    }
+}
+// appends one projection's blocks to the launch
+static void gemm_seg(GemmArgs &a, const DMat &m, float *c, const GemmPlan &p, int rows_per_tile, int &blocks) {
+    const int nchunk = m.cols / GM_KC, nx = gemm_rt(m, rows_per_tile);
+    a.seg[a.nseg++] = GemmSeg{m, c, (nchunk + p.split - 1) / p.split, nx, blocks};
+    blocks += nx * ((a.n + 16 * p.tt - 1) / (16 * p.tt)) * p.split;
 }
 
 // With split > 1 the slices' partial products go to `part` (split * n * rows
@@ -490,16 +605,15 @@ int gemm_split(const DMat &m, int32_t n, size_t part_bytes) {
 hipError_t launch_gemm(const DMat &m, const uint16_t *x, int32_t n, float *c, float *part, size_t part_bytes,
                        hipStream_t st) {
     if (!gemm_supported(m) || n <= 0) return hipErrorInvalidValue;
-    const int nchunk = m.cols / GM_KC;
-    const int split = gemm_split(m, n, part ? part_bytes : 0);
-    const int cps = (nchunk + split - 1) / split;
-    GemmArgs a{m, x, split > 1 ? part : c, n, DMat{}, nullptr, 0, {}};
-    dim3 grid((m.rows + GM_ROWS - 1) / GM_ROWS, (n + GM_TOK - 1) / GM_TOK, split), block(GM_THREADS);
-    switch (m.type) {
-    case T_Q4_K: hipLaunchKernelGGL(gemm_q_kernel<GQ4K>, grid, block, 0, st, a, cps); break;
-    case T_Q6_K: hipLaunchKernelGGL(gemm_q_kernel<GQ6K>, grid, block, 0, st, a, cps); break;
-    default: hipLaunchKernelGGL(gemm_q_kernel<GQ80>, grid, block, 0, st, a, cps); break;
-    }
+    const GemmPlan p = gemm_plan(m, n, part ? part_bytes : 0);
+    const int split = p.split;
+    GemmArgs a{};
+    a.x = x;
+    a.n = n;
+    int blocks = 0;
+    gemm_seg(a, m, split > 1 ? part : c, p, GM_ROWS, blocks);
+    const hipError_t r = gemm_launch<1>(a, blocks, p.tt, st);
+    if (r != hipSuccess) return r;
     if (split > 1) {
         const int64_t total = (int64_t)n * m.rows;
         const int64_t nb = ((total + 3) / 4 + WG - 1) / WG;
@@ -508,72 +622,61 @@ hipError_t launch_gemm(const DMat &m, const uint16_t *x, int32_t n, float *c, fl
     return hipGetLastError();
 }
 
-// h[t][r] = f16(silu(gate x)[t][r] * (up x)[t][r]) in one pass over K: only
-// when the projection needs no K split (gemm_split == 1 for this n)
+// h[t][r] = f16(silu(gate x)[t][r] * (up x)[t][r]) in one pass over K: worth it
+// where its tiles, which cannot split K, fill half of the CUs
 bool gemm_swiglu_supported(const DMat &gate, const DMat &up, int32_t n) {
-    return gemm_supported(gate) && up.type == gate.type && up.rows == gate.rows && up.cols == gate.cols && n > 0 &&
-           gemm_split(gate, n, SIZE_MAX) == 1;
+    if (!gemm_supported(gate) || up.type != gate.type || up.rows != gate.rows || up.cols != gate.cols || n <= 0) return false;
+    const int rt = gemm_rt(gate, GM_ROWS / 2);
+    return rt * ((n + 127) / 128) >= 128;
 }
 
 hipError_t launch_gemm_swiglu(const DMat &gate, const DMat &up, const uint16_t *x, int32_t n, uint16_t *h,
                               hipStream_t st) {
     if (!gemm_swiglu_supported(gate, up, n) || !h) return hipErrorInvalidValue;
-    GemmArgs a{gate, x, nullptr, n, up, h, 0, {}};
-    dim3 grid((gate.rows + GM_ROWS - 1) / GM_ROWS, (n + GM_TOK - 1) / GM_TOK, 1), block(GM_THREADS);
-    const int cps = gate.cols / GM_KC;
-    switch (gate.type) {
-    case T_Q4_K: hipLaunchKernelGGL((gemm_q_kernel<GQ4K, 2>), grid, block, 0, st, a, cps); break;
-    case T_Q6_K: hipLaunchKernelGGL((gemm_q_kernel<GQ6K, 2>), grid, block, 0, st, a, cps); break;
-    default: hipLaunchKernelGGL((gemm_q_kernel<GQ80, 2>), grid, block, 0, st, a, cps); break;
-    }
-    return hipGetLastError();
+    GemmArgs a{};
+    a.x = x;
+    a.n = n;
+    a.m2 = up;
+    a.h = h;
+    const GemmPlan p = gemm_plan(gate.type, gemm_rt(gate, GM_ROWS / 2), gate.cols / GM_KC, n, 0.0, 1, false);
+    int blocks = 0;
+    gemm_seg(a, gate, nullptr, p, GM_ROWS / 2, blocks);
+    return gemm_launch<2>(a, blocks, p.tt, st);
 }
 
 hipError_t launch_gemm_parts(const DMat &m, const uint16_t *x, int32_t n, float *part, size_t part_bytes, int *split,
                              hipStream_t st) {
-    if (!gemm_supported(m) || n <= 0 || !part || part_bytes < (size_t)n * m.rows * 4) return hipErrorInvalidValue;
-    const int nchunk = m.cols / GM_KC;
-    *split = gemm_split(m, n, part_bytes);
-    const int cps = (nchunk + *split - 1) / *split;
-    GemmArgs a{m, x, part, n, DMat{}, nullptr, 0, {}};
-    dim3 grid((m.rows + GM_ROWS - 1) / GM_ROWS, (n + GM_TOK - 1) / GM_TOK, *split), block(GM_THREADS);
-    switch (m.type) {
-    case T_Q4_K: hipLaunchKernelGGL(gemm_q_kernel<GQ4K>, grid, block, 0, st, a, cps); break;
-    case T_Q6_K: hipLaunchKernelGGL(gemm_q_kernel<GQ6K>, grid, block, 0, st, a, cps); break;
-    default: hipLaunchKernelGGL(gemm_q_kernel<GQ80>, grid, block, 0, st, a, cps); break;
-    }
-    return hipGetLastError();
+    const DMat *ms[1] = {&m};
+    return launch_gemm_parts_multi(ms, &part, &part_bytes, 1, x, n, split, st);
 }
 
-// launch_gemm_parts for up to GM_MAX_SEG projections of the same x in one
-// launch (same type and K): the same blocks, K slices and partial products as
-// one launch each, so the same results; one launch's fixed cost instead of
-// nseg (the DeltaNet layer's four input projections at 64 tokens: 28.7 us in
-// four launches)
+// up to GM_MAX_SEG projections of the same x in one launch (same type and K):
+// one launch's fixed cost instead of nseg (the DeltaNet layer's four input
+// projections at 64 tokens: 28.7 us in four launches), and one plan for all of
+// them, chosen for the launch's blocks together
 hipError_t launch_gemm_parts_multi(const DMat *const *m, float *const *part, const size_t *part_bytes, int nseg,
                                    const uint16_t *x, int32_t n, int *split, hipStream_t st) {
     if (nseg < 1 || nseg > GM_MAX_SEG || n <= 0) return hipErrorInvalidValue;
-    GemmArgs a{*m[0], x, nullptr, n, DMat{}, nullptr, nseg, {}};
-    int blocks = 0;
-    const int ny = (n + GM_TOK - 1) / GM_TOK;
+    int rt = 0, cap = 64;
+    double out = 0;
     for (int i = 0; i < nseg; i++) {
-        const DMat &mi = *m[i];
-        if (!gemm_supported(mi) || mi.type != m[0]->type || mi.cols != m[0]->cols || !part[i] ||
-            part_bytes[i] < (size_t)n * mi.rows * 4)
+        if (!gemm_supported(*m[i]) || m[i]->type != m[0]->type || m[i]->cols != m[0]->cols || !part[i] ||
+            part_bytes[i] < (size_t)n * m[i]->rows * 4)
             return hipErrorInvalidValue;
-        const int nchunk = mi.cols / GM_KC;
-        split[i] = gemm_split(mi, n, part_bytes[i]);
-        const int nx = (mi.rows + GM_ROWS - 1) / GM_ROWS;
-        a.seg[i] = GemmSeg{mi, part[i], (nchunk + split[i] - 1) / split[i], nx, blocks};
-        blocks += nx * ny * split[i];
+        rt += gemm_rt(*m[i]);
+        out += (double)n * m[i]->rows;
+        cap = std::min(cap, gemm_cap(*m[i], n, part_bytes[i]));
     }
-    const dim3 grid((unsigned)blocks), block(GM_THREADS);
-    switch (m[0]->type) {
-    case T_Q4_K: hipLaunchKernelGGL(gemm_q_kernel<GQ4K>, grid, block, 0, st, a, 0); break;
-    case T_Q6_K: hipLaunchKernelGGL(gemm_q_kernel<GQ6K>, grid, block, 0, st, a, 0); break;
-    default: hipLaunchKernelGGL(gemm_q_kernel<GQ80>, grid, block, 0, st, a, 0); break;
+    const GemmPlan p = gemm_plan(m[0]->type, rt, m[0]->cols / GM_KC, n, out, cap, false);
+    GemmArgs a{};
+    a.x = x;
+    a.n = n;
+    int blocks = 0;
+    for (int i = 0; i < nseg; i++) {
+        split[i] = p.split;
+        gemm_seg(a, *m[i], part[i], p, GM_ROWS, blocks);
     }
-    return hipGetLastError();
+    return gemm_launch<1>(a, blocks, p.tt, st);
 }
 
 }  // namespace oi

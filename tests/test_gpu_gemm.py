@@ -172,3 +172,18 @@ def test_gemm_workspace_split(kind, m, n, k):
     assert np.array_equal(split1, split2)
     for got in (split1, whole, fewer):
         assert scaled_err(got, ref) <= 1e-2
+
+
+@pytest.mark.parametrize("kind", [12, 14, 8])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 256), (127, 31, 256), (129, 33, 512), (130, 64, 768), (256, 65, 512),
+                                   (40, 127, 1280), (132, 129, 256), (128, 200, 2304), (70, 300, 512)])
+def test_gemm_tile_edges(kind, m, n, k):
+    """One past and one short of the tiles (128 rows; 32, 64 and 128 tokens; chunks
+    of 256 in K halves; rows not a multiple of 4): f32 sums of exact products differ
+    from the float64 sum by at most K 2^-24 sum|w x|, and sum|w x| is about sqrt(K)
+    times the result's size for these random signs."""
+    rng = np.random.default_rng(m * 31 + n * 7 + k + kind)
+    w = gemm_blocks(kind, m, k, rng)
+    x = x16(rng.uniform(-1, 1, size=(n, k)))
+    err = scaled_err(ggml.gemm(kind, w, m, k, x), refcpu.gemm_f16(w, kind, m, k, x))
+    assert err <= k ** 1.5 * 2.0 ** -24, "%d %dx%dx%d scaled error %.3g" % (kind, m, n, k, err)
