@@ -1456,16 +1456,16 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
             PfQkvArgs qa{P[0], P[1], P[2], qs, ks, vs, L.q_norm, L.k_norm, eps, e->rope_cs, L.kc, L.vc, e->pf_q,
                          T, pos, (int32_t)c.seq_len, (int32_t)c.n_heads, (int32_t)c.n_kv_heads};
             HIP_TRY(launch_pf_qkv(qa, hd, st));
+            // the k / v partial products are consumed: their buffer is the
+            // attention's scratch
             HIP_TRY(launch_pf_attn(e->pf_q, L.kc, L.vc, e->pf_xb, T, pos, (int)c.seq_len, (int)c.n_heads,
-                                   (int)c.n_kv_heads, hd, st));
+                                   (int)c.n_kv_heads, hd, st, nullptr, P[1], PB[1]));
             HIP_TRY(launch_gemm_parts(L.wo, e->pf_xb, T, P[0], PB[0], &s0, st));
         } else if (L.kind == LK_FULL) {
             PfQ35Args qa{P[0], P[1], P[2], qs, ks, vs, L.q_norm, L.k_norm, e->inv_freq, eps, (int32_t)e->rotary_dim,
                          L.kc, L.vc, e->pf_q, e->pf_gate, T, pos, (int32_t)c.seq_len, (int32_t)c.n_heads,
                          (int32_t)c.n_kv_heads};
             HIP_TRY(launch_pf_q35_qkv(qa, hd, st));
-            // the k / v partial products are consumed: their buffer is the
-            // attention's scratch
             HIP_TRY(launch_pf_attn(e->pf_q, L.kc, L.vc, e->pf_xb, T, pos, (int)c.seq_len, (int)c.n_heads,
                                    (int)c.n_kv_heads, hd, st, e->pf_gate, P[1], PB[1]));
             HIP_TRY(launch_gemm_parts(L.wo, e->pf_xb, T, P[0], PB[0], &s0, st));

@@ -305,8 +305,9 @@ __global__ __launch_bounds__(WG) void pf_attn_kernel(PfAttnArgs a) {
 // Causal attention on the matrix cores for head_dim 128 or 256, grid (n_heads,
 // ceil(T / 64)): a workgroup takes 64 queries of one head (wave w: queries
 // 16w .. 16w+15) and walks the keys in blocks of 64 up to its last query's
-// position.  Per block, K (rows padded to HD + 8 halves) and V transposed (V^T,
-// rows of 68 halves) are staged in LDS; then per wave
+// position.  Per block, K (rows padded to HD + 8 halves) and V transposed (V^T)
+// are staged in LDS, the next block's rows already on their way in registers;
+// then per wave
 //   S^T[key][query] = K Q^T  (v_mfma_f32_16x16x32_f16; A = K rows, B = Q),
 //   online softmax per query (running max, exp, running sum),
 //   O^T[d][query] += V^T P^T (A = V^T rows, B = P).
@@ -317,7 +318,13 @@ __global__ __launch_bounds__(WG) void pf_attn_kernel(PfAttnArgs a) {
 // split into f16 hi + lo halves (two products each), K and V are exact f16,
 // accumulation is f32, so scores and weights keep about 22 bits, close to the
 // reference's f32 arithmetic (infer/forward.odin:87-115).
-constexpr int FA_VP = 68;  // LDS row stride (halves) of V^T; K rows: HD + 8
+//
+// V^T: row d is 16 groups of four keys (8 bytes); group kg is stored at kg ^ ((d /
+// 2) % 16), which spreads both the transposing stores (a thread has four keys x
+// eight d: eight 8-byte stores where single halves took 32 2-byte ones, four lanes
+// to a bank) and the operand reads evenly over the banks.
+constexpr int FA_VG = 16;  // key groups per V^T row
+static __device__ __forceinline__ int fa_vslot(int d, int kg) { return d * FA_VG + (kg ^ ((d >> 1) & 15)); }
 
 static __device__ __forceinline__ void split16(const float (&v)[8], h8 &hi, h8 &lo) {
 #pragma unroll
@@ -334,8 +341,9 @@ static __device__ __forceinline__ void split16(const float (&v)[8], h8 &hi, h8 &
 template <int HD, bool SPLIT = false>
 __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float *ws = nullptr) {
     constexpr int FA_KP = HD + 8, NC = HD / 32, NDT = HD / 16;  // K row stride; 32-wide K chunks; 16-wide d tiles
+    constexpr int KPT = HD / 32, VPT = HD / 128;  // per thread and block: 16-byte K pieces; (4 keys x 8 d) V tiles
     __shared__ __attribute__((aligned(16))) uint16_t ks[64 * FA_KP];
-    __shared__ __attribute__((aligned(16))) uint16_t vt[HD * FA_VP];
+    __shared__ __attribute__((aligned(16))) u32x2 vt[HD * FA_VG];
     const int h = blockIdx.x, t0 = 64 * (int)blockIdx.y;
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     const int q = lane & 15, g = lane >> 4;
@@ -371,21 +379,43 @@ __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float
         kb0 = (int)((long)nb * z / ns);
         kb1 = (int)((long)nb * (z + 1) / ns);
     }
-    for (int kb = kb0; kb < kb1; kb++) {
-        // stage K and V^T of keys 64 kb .. +63 (rows past the written range
-        // re-read the last written row; their scores are masked)
-        __syncthreads();
+    // a block's K pieces and V tiles of this thread (rows past the written range
+    // re-read the last written row; their scores are masked)
+    u32x4 kr[KPT], vr[VPT][4];
+    auto fetch = [&](int kb) {
 #pragma unroll
-        for (int i = 0; i < 64 * (HD / 8) / WG; i++) {
+        for (int i = 0; i < KPT; i++) {
             const int piece = threadIdx.x + WG * i, r = piece / (HD / 8), c8 = piece % (HD / 8);  // row r, 8 halves at 8 c8
-            const int p = min(64 * kb + r, lmax - 1);
-            const u32x4 kv = *(const u32x4 *)(kc + (size_t)p * HD + 8 * c8);
-            *(u32x4 *)(ks + r * FA_KP + 8 * c8) = kv;
-            const u32x4 vv = *(const u32x4 *)(vc + (size_t)p * HD + 8 * c8);
+            kr[i] = *(const u32x4 *)(kc + (size_t)min(64 * kb + r, lmax - 1) * HD + 8 * c8);
+        }
 #pragma unroll
-            for (int e = 0; e < 8; e++) vt[(8 * c8 + e) * FA_VP + r] = (uint16_t)((vv[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
+        for (int i = 0; i < VPT; i++) {
+            const int piece = threadIdx.x + WG * i, kg = piece / (HD / 8), c8 = piece % (HD / 8);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                vr[i][j] = *(const u32x4 *)(vc + (size_t)min(64 * kb + 4 * kg + j, lmax - 1) * HD + 8 * c8);
+        }
+    };
+    if (kb0 < kb1) fetch(kb0);
+    for (int kb = kb0; kb < kb1; kb++) {
+        __syncthreads();  // the previous block has been read
+#pragma unroll
+        for (int i = 0; i < KPT; i++) {
+            const int piece = threadIdx.x + WG * i, r = piece / (HD / 8), c8 = piece % (HD / 8);
+            *(u32x4 *)(ks + r * FA_KP + 8 * c8) = kr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < VPT; i++) {
+            const int piece = threadIdx.x + WG * i, kg = piece / (HD / 8), c8 = piece % (HD / 8);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {  // halves e of the four keys
+                const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+                vt[fa_vslot(8 * c8 + e, kg)] = u32x2{__builtin_amdgcn_perm(vr[i][1][e >> 1], vr[i][0][e >> 1], sel),
+                                                     __builtin_amdgcn_perm(vr[i][3][e >> 1], vr[i][2][e >> 1], sel)};
+            }
         }
         __syncthreads();
+        if (kb + 1 < kb1) fetch(kb + 1);
         // S^T tiles kt (keys 16 kt + 4g + e for query q)
         float s[4][4];
 #pragma unroll
@@ -438,8 +468,7 @@ __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float
             split16(pv, ph, pl);
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++) {
-                const uint16_t *vr = vt + (16 * dt + q) * FA_VP + 32 * kc2 + 4 * g;
-                const u32x2 v0 = *(const u32x2 *)vr, v1 = *(const u32x2 *)(vr + 16);
+                const u32x2 v0 = vt[fa_vslot(16 * dt + q, 8 * kc2 + g)], v1 = vt[fa_vslot(16 * dt + q, 8 * kc2 + 4 + g)];
                 const h8 vA = __builtin_bit_cast(h8, u32x4{v0.x, v0.y, v1.x, v1.y});
                 o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vA, ph, o[dt], 0, 0, 0);
                 o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vA, pl, o[dt], 0, 0, 0);
@@ -475,24 +504,46 @@ __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float
     }
 }
 
-// The splits of pf_fattn_kernel<HD, true> for token t and head h (grid (T,
-// n_heads), thread d): O = sum_s e^{m_s - M} o_s / sum_s e^{m_s - M} l_s.
+// The splits of pf_fattn_kernel<HD, true>, a wave per (token, head) pair p = t
+// n_heads + h: O = sum_s e^{m_s - M} o_s / sum_s e^{m_s - M} l_s.  Lane z holds split
+// z's m and l (at most 64 splits); the weighted sums of the lane's HD / 64 dimensions run over
+// four splits' loads at a time.
 template <int HD>
-__global__ __launch_bounds__(HD) void pf_fattn_merge_kernel(PfAttnArgs a, int T, const float *ws, int ns) {
+__global__ __launch_bounds__(WG) void pf_fattn_merge_kernel(PfAttnArgs a, int T, const float *ws, int ns) {
 #pragma clang fp contract(off)
-    const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x, QD = a.n_heads * HD;
-    const size_t stride = (size_t)T * a.n_heads * (HD + 2), base = ((size_t)t * a.n_heads + h) * (HD + 2);
-    float M = -INFINITY;
-    for (int z = 0; z < ns; z++) M = fmaxf(M, ws[z * stride + base + HD]);
-    float L = 0.f, O = 0.f;
-    for (int z = 0; z < ns; z++) {
-        const float mz = ws[z * stride + base + HD];
-        const float f = mz == -INFINITY ? 0.f : expf(mz - M);  // a split with no visible key adds nothing
-        L += f * ws[z * stride + base + HD + 1];
-        O += f * ws[z * stride + base + d];
+    constexpr int DPL = HD / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), p = (int)blockIdx.x * (WG / WAVE) + (int)threadIdx.x / WAVE;
+    if (p >= T * a.n_heads) return;
+    const size_t stride = (size_t)T * a.n_heads * (HD + 2), base = (size_t)p * (HD + 2);
+    float mz = -INFINITY, lz = 0.f;
+    if (lane < ns) {
+        mz = ws[lane * stride + base + HD];
+        lz = ws[lane * stride + base + HD + 1];
     }
-    const size_t i = (size_t)t * QD + h * HD + d;
-    a.out[i] = f2h(pf_gated(a, O / L, i));
+    const float M = wave_max_all(mz);
+    const float f = mz == -INFINITY ? 0.f : expf(mz - M);  // a split with no visible key adds nothing
+    const float L = wave_sum(f * lz);
+    float O[DPL];
+#pragma unroll
+    for (int e = 0; e < DPL; e++) O[e] = 0.f;
+    for (int z0 = 0; z0 < ns; z0 += 4) {
+        float v[4][DPL];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int e = 0; e < DPL; e++) v[k][e] = ws[(size_t)min(z0 + k, ns - 1) * stride + base + lane + WAVE * e];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float fz = z0 + k < ns ? lane_value(f, z0 + k) : 0.f;
+#pragma unroll
+            for (int e = 0; e < DPL; e++) O[e] += fz * v[k][e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < DPL; e++) {
+        const size_t i = (size_t)p * HD + lane + WAVE * e;
+        a.out[i] = f2h(pf_gated(a, O[e] / L, i));
+    }
 }
 
 // x[i] += sum of the partial products of element i (the residual adds,
@@ -537,18 +588,24 @@ hipError_t launch_pf_attn(const float *q, const uint16_t *kc, const uint16_t *vc
     PfAttnArgs a{q, kc, vc, out, pos0, seq_len, n_heads, n_kv_heads, gate};
     const dim3 grid((unsigned)n_heads, (unsigned)T);
     const dim3 fgrid((unsigned)n_heads, (unsigned)((T + 63) / 64));
-    // a short chunk at head_dim 256: the key blocks split over workgroups (up
-    // to 16 per query tile, at least 2 blocks each) when the workspace holds
-    // the partials
-    const int nkb = (pos0 + T + 63) / 64, qt = (T + 63) / 64;
+    // The key blocks of a query tile are split over workgroups where the tiles
+    // alone do not fill the GPU twice (45 tokens of 32 heads after 3000 positions: 32
+    // workgroups walked 48 blocks each, 181 us a layer; 512 workgroups of 3 blocks
+    // take a tenth), each split at least 2 blocks, when the workspace holds the
+    // partial results.
+    const int nkb = (pos0 + T + 63) / 64, qt = (T + 63) / 64, wgs = qt * n_heads;
     const size_t per = (size_t)T * n_heads * (head_dim + 2) * 4;
-    int ns = std::min(16, nkb / 2);
-    if (ws && per > 0) ns = std::min<int>(ns, (int)(ws_bytes / per));
-    if (head_dim == 256 && T < 128 && !pf_attn_lanes() && ws && ns >= 2 && qt * n_heads < 256) {
-        hipLaunchKernelGGL((pf_fattn_kernel<256, true>), dim3((unsigned)n_heads, (unsigned)qt, (unsigned)ns), dim3(WG),
-                           0, st, a, T, ws);
-        hipLaunchKernelGGL(pf_fattn_merge_kernel<256>, dim3((unsigned)T, (unsigned)n_heads), dim3(256), 0, st, a, T,
-                           (const float *)ws, ns);
+    int ns = std::min({16, nkb / 2, (512 + wgs - 1) / wgs});
+    if (ws && per > 0) ns = std::min<int>(ns, (int)std::min<size_t>(ws_bytes / per, 16));
+    if ((head_dim == 128 || head_dim == 256) && !(head_dim == 256 && pf_attn_lanes()) && ws && ns >= 2) {
+        const dim3 sgrid((unsigned)n_heads, (unsigned)qt, (unsigned)ns), mgrid((unsigned)((T * n_heads + WG / WAVE - 1) / (WG / WAVE)));
+        if (head_dim == 128) {
+            hipLaunchKernelGGL((pf_fattn_kernel<128, true>), sgrid, dim3(WG), 0, st, a, T, ws);
+            hipLaunchKernelGGL(pf_fattn_merge_kernel<128>, mgrid, dim3(WG), 0, st, a, T, (const float *)ws, ns);
+        } else {
+            hipLaunchKernelGGL((pf_fattn_kernel<256, true>), sgrid, dim3(WG), 0, st, a, T, ws);
+            hipLaunchKernelGGL(pf_fattn_merge_kernel<256>, mgrid, dim3(WG), 0, st, a, T, (const float *)ws, ns);
+        }
         return hipGetLastError();
     }
     if (head_dim == 128) hipLaunchKernelGGL((pf_fattn_kernel<128>), fgrid, dim3(WG), 0, st, a, T, nullptr);

@@ -182,3 +182,22 @@ def test_prefill_errors(make_model):
         assert np.isfinite(infer.engine_forward_batch(e, np.arange(8, dtype=np.int32), 0)).all()
     finally:
         infer.engine_destroy(e)
+
+
+@pytest.mark.parametrize("name", ["tiny-q4_k", "tiny-q8_0"])
+@pytest.mark.parametrize("n", [8, 40, 72, 136])
+def test_prefill_chunk_after_a_long_prompt(make_model, name, n):
+    """A chunk after 600 positions: its key blocks are split over workgroups and
+    merged (one, one, two and three query tiles, the last ones ragged)."""
+    path = make_model(name)
+    e, r = _engines(path, 1024)
+    try:
+        toks = _tokens(600 + n, 600 + n, r.vocab_size)
+        infer.engine_forward_batch(e, toks[:600], 0)
+        r.prefill(toks[:600], 0)
+        got = infer.engine_forward_batch(e, toks[600:], 600).copy()
+        err = scaled_err(got, r.prefill(toks[600:], 600))
+        assert err <= TOL, "scaled error %.3g" % err
+    finally:
+        infer.engine_destroy(e)
+        r.close()
