@@ -94,7 +94,7 @@ const float *oi_engine_forward(oi_engine *e, int32_t token, int32_t pos);
  * batched: the seven projections of each layer on the matrix cores with f16
  * operands and f32 accumulation (the reference's MMQ), the per-token operations
  * (norms, RoPE, cache store, causal attention, SwiGLU, residuals) in f32; the
- * trailing 1-7 tokens go through oi_engine_forward's path.  A model whose
+ * trailing 1-7 tokens in oi_engine_forward's f32 arithmetic.  A model whose
  * projections the batched kernels cannot take (type other than Q4_K / Q6_K /
  * Q8_0, or a row length not a multiple of 256) runs every token through that
  * path, as the reference's non-Metal fallback (qwen3_5/engine.odin:86-91).  NULL on

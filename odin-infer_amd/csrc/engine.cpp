@@ -1431,6 +1431,40 @@ int prefill_projections(oi_engine *e, const DMat *const *m, const int *idx, int 
     return OI_OK;
 }
 
+// The final RMSNorm and classifier of pf_x rows [t0, t0 + n) in f32 (the token
+// step's arithmetic, each row's result the same in any group), row i's logits to
+// out + i * vocab: up to GEMV_NT_MAX rows per pass over the classifier, which was
+// read once for every row (151936 x 4096 Q6_K: 79 us a row).
+static int prefill_classify(oi_engine *e, int t0, int n, float *out) {
+    const int D = (int)e->cfg.dim;
+    const size_t V = (size_t)e->cfg.vocab_size;
+    const int group = gemv_nt_supported(e->output) ? GEMV_NT_MAX : 1;
+    for (int i = 0; i < n; i += group) {
+        const float *x = e->pf_x + (size_t)(t0 + i) * D;
+        if (group > 1) {
+            GemvNtArgs a{};
+            a.nseg = 1;
+            a.mode = GEMV_STORE;
+            a.n = std::min(group, n - i);
+            a.K = D;
+            a.x = x;
+            a.norm_w = e->output_norm;
+            a.eps = e->cfg.rms_eps;
+            a.seg[0].m = e->output;
+            a.seg[0].y = out + (size_t)i * V;
+            HIP_TRY(launch_gemv_nt(a, e->stream));
+            continue;
+        }
+        GemvArgs a = gemv_args(GEMV_STORE, D, x, e->output_norm, e->cfg.rms_eps);
+        a.nseg = 1;
+        a.seg[0].m = e->output;
+        a.seg[0].y = out + (size_t)i * V;
+        if (!plan_gemv(a)) return fail(OI_E_DEVICE, "internal: classifier plan");
+        HIP_TRY(launch_gemv(a, e->stream));
+    }
+    return OI_OK;
+}
+
 int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *rows = nullptr) {
     const hipStream_t st = e->stream;
     const oi_config &c = e->cfg;
@@ -1526,17 +1560,90 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
             HIP_TRY(launch_pf_add(e->pf_x, P[0], s0, (int64_t)T * D, st));
     }
     // the final norm and classifier (qwen3_5/metal.odin:1637-1641 for the last token;
-    // metal_verify_batch_logits, qwen3_5/metal.odin:1707-1747, for every token): the
-    // decode path's f32 GEMV with the RMSNorm prologue, one row at a time
-    for (int t = rows ? 0 : T - 1; t < T; t++) {
-        GemvArgs a = gemv_args(GEMV_STORE, D, e->pf_x + (size_t)t * D, e->output_norm, eps);
-        a.nseg = 1;
-        a.seg[0].m = e->output;
-        a.seg[0].y = rows ? rows + (size_t)t * c.vocab_size : e->logits;
-        if (!plan_gemv(a)) return fail(OI_E_DEVICE, "internal: classifier plan");
-        HIP_TRY(launch_gemv(a, st));
-    }
+    // metal_verify_batch_logits, qwen3_5/metal.odin:1707-1747, for every token)
+    if (rows) return prefill_classify(e, 0, T, rows);
+    GemvArgs a = gemv_args(GEMV_STORE, D, e->pf_x + (size_t)(T - 1) * D, e->output_norm, eps);
+    a.nseg = 1;
+    a.seg[0].m = e->output;
+    a.seg[0].y = e->logits;
+    if (!plan_gemv(a)) return fail(OI_E_DEVICE, "internal: classifier plan");
+    HIP_TRY(launch_gemv(a, st));
     return OI_OK;
+}
+
+// The trailing 2-7 tokens of a call in one pass over the layers, in the arithmetic
+// of the token step (f32 activations, nothing staged in half): its GEMVs for all
+// the tokens at once (launch_gemv_nt), the chunk's attention, DeltaNet (token by
+// token) and routed experts between them.  Each trailing token through the token
+// step reads every weight again: five tokens of the 8B shape took 5 x 1.85 ms.
+int prefill_few(oi_engine *e, const int32_t *tokens, int T, int pos, float *rows) {
+    const hipStream_t st = e->stream;
+    const oi_config &c = e->cfg;
+    const int D = (int)c.dim, hd = (int)c.head_dim;
+    float *const *P = e->pf_p;
+    const size_t *PB = e->pf_pbytes;
+    float *act = (float *)e->pf_xb;  // the attention's or DeltaNet's f32 output rows
+    HIP_TRY(hipMemcpyAsync(e->pf_tok, tokens, (size_t)T * 4, hipMemcpyHostToDevice, st));
+    HIP_TRY(launch_embed_rows(e->tok_embd, e->pf_tok, T, e->pf_x, st));
+    auto nt = [&](int mode, const float *x, const float *norm, std::initializer_list<std::pair<const DMat *, float *>> ms) {
+        GemvNtArgs a{};
+        a.mode = mode;
+        a.n = T;
+        a.K = ms.begin()->first->cols;
+        a.x = x;
+        a.norm_w = norm;
+        a.eps = c.rms_eps;
+        for (const auto &m : ms) {
+            a.seg[a.nseg].m = *m.first;
+            a.seg[a.nseg++].y = m.second;
+        }
+        return launch_gemv_nt(a, st);
+    };
+    for (const LayerDev &L : e->layers) {
+        if (L.kind == LK_LINEAR) {
+            HIP_TRY(nt(GEMV_STORE, e->pf_x, L.attn_norm, {{&L.in_qkv, P[0]}, {&L.in_z, P[1]}, {&L.in_b, P[2]}, {&L.in_a, P[3]}}));
+            PfDnArgs da{};
+            da.qkv = P[0]; da.z = P[1]; da.b = P[2]; da.a = P[3];
+            da.qkvs = da.zs = da.bs = da.as = 1;
+            da.conv_w = L.conv_w; da.a_decay = L.ssm_a; da.dt_bias = L.dt_bias; da.norm_w = L.ssm_norm;
+            da.eps = c.rms_eps;
+            da.conv_state = L.conv_state;
+            da.state = L.rec_state;
+            da.conv_out = e->pf_conv; da.qk = e->pf_qk; da.gates = e->pf_gates; da.o = e->pf_o;
+            da.out32 = act;
+            da.T = T;
+            da.n_kh = (int32_t)e->lin_nk; da.n_vh = (int32_t)e->lin_nv;
+            da.hk = (int32_t)e->lin_hk; da.hv = (int32_t)e->lin_hv; da.kernel = (int32_t)e->lin_kernel;
+            HIP_TRY(launch_pf_deltanet(da, st));
+            HIP_TRY(nt(GEMV_ADD, act, nullptr, {{&L.ssm_out, e->pf_x}}));
+        } else {
+            HIP_TRY(nt(GEMV_STORE, e->pf_x, L.attn_norm, {{&L.wq, P[0]}, {&L.wk, P[1]}, {&L.wv, P[2]}}));
+            if (L.kind == LK_QWEN3) {
+                PfQkvArgs qa{P[0], P[1], P[2], 1, 1, 1, L.q_norm, L.k_norm, c.rms_eps, e->rope_cs, L.kc, L.vc, e->pf_q,
+                             T, pos, (int32_t)c.seq_len, (int32_t)c.n_heads, (int32_t)c.n_kv_heads};
+                HIP_TRY(launch_pf_qkv(qa, hd, st));
+            } else {
+                PfQ35Args qa{P[0], P[1], P[2], 1, 1, 1, L.q_norm, L.k_norm, e->inv_freq, c.rms_eps, (int32_t)e->rotary_dim,
+                             L.kc, L.vc, e->pf_q, e->pf_gate, T, pos, (int32_t)c.seq_len, (int32_t)c.n_heads,
+                             (int32_t)c.n_kv_heads};
+                HIP_TRY(launch_pf_q35_qkv(qa, hd, st));
+            }
+            HIP_TRY(launch_pf_attn(e->pf_q, L.kc, L.vc, nullptr, T, pos, (int)c.seq_len, (int)c.n_heads, (int)c.n_kv_heads,
+                                   hd, st, L.kind == LK_FULL ? e->pf_gate : nullptr, P[1], PB[1], act));
+            HIP_TRY(nt(GEMV_ADD, act, nullptr, {{&L.wo, e->pf_x}}));
+        }
+        if (L.moe) {
+            const bool xq = pf_xq_used(e);
+            HIP_TRY(launch_pf_addnorm16(e->pf_x, nullptr, 1, L.ffn_norm, c.rms_eps, D, T, e->pf_xb, st, e->pf_xn, nullptr,
+                                        nullptr, 0, xq ? e->pf_xq : nullptr, e->pf_xq_sum, e->pf_xq_scale));
+            if (prefill_moe(e, L, T)) return -1;
+            HIP_TRY(launch_pf_add(e->pf_x, P[0], 1, (int64_t)T * D, st));
+        } else {
+            HIP_TRY(nt(GEMV_SWIGLU, e->pf_x, L.ffn_norm, {{&L.w1, P[1]}, {&L.w3, nullptr}}));
+            HIP_TRY(nt(GEMV_ADD, P[1], nullptr, {{&L.w2, e->pf_x}}));
+        }
+    }
+    return rows ? prefill_classify(e, 0, T, rows) : prefill_classify(e, T - 1, 1, e->logits);
 }
 
 }  // namespace
@@ -1544,7 +1651,7 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
 namespace {
 
 // engine_forward_batch over tokens[0, n) at pos0 (chunks of a multiple of 8
-// up to PF_MAX_T batched, the trailing 1-7 through the decode path).  rows ==
+// up to PF_MAX_T batched, the trailing 1-7 in the decode path's arithmetic).  rows ==
 // nullptr: the last token's logits in e->logits; otherwise every token's
 // logits, token i at rows + i * vocab (device memory).  Returns 0 or a code.
 int prefill_run(oi_engine *e, const int32_t *tokens, int32_t n, int32_t pos0, float *rows) {
@@ -1571,6 +1678,9 @@ int prefill_run(oi_engine *e, const int32_t *tokens, int32_t n, int32_t pos0, fl
             chunk -= chunk % 8;
             if (prefill_chunk(e, tokens + i, chunk, pos0 + i, rows ? rows + (size_t)i * V : nullptr)) return -1;
             i += chunk;
+        } else if (batched && rem >= (e->lin_nv > 0 ? (int)e->lin_kernel - 1 : 2)) {  // the trailing tokens at once
+            if (prefill_few(e, tokens + i, rem, pos0 + i, rows ? rows + (size_t)i * V : nullptr)) return -1;
+            i += rem;
         } else {  // one token through the decode path
             if (set_state(e, tokens[i], pos0 + i, 0) || run_token(e)) return -1;
             hipError_t r = hipSuccess;

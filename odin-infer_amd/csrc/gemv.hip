@@ -1142,6 +1142,257 @@ hipError_t launch_gemv_q(const GemvArgs &a, hipStream_t st) {
     return hipSuccess;
 }
 
+// -------------------------------------------- a few tokens at once
+// gemv_nt_kernel: the GEMV above for n <= GEMV_NT_MAX tokens.  A prompt's trailing
+// tokens, a draft of a few tokens and the classifier of every position read the
+// same weights for each token; here a lane's unit is loaded and held once and
+// dotted with every token's x in turn, in the token step's arithmetic (quant4's
+// planes, v_dot4_i32_i8, the same scaling), so each token's result is as exact as
+// alone.
+//
+// One workgroup of 8 waves per CU takes a contiguous range of row tiles (R rows
+// per lane group) of one segment; all tokens' planes sit in LDS (14 KB a token
+// at 4096 columns).  Longer rows run in passes of ks columns, the results kept in
+// LDS between them.  Lanes per row is the power of two that covers a pass's units;
+// lanes past them read its last unit and add nothing.  What bounds it: the weights
+// below 3 tokens, then the products (64 vector instructions per unit and token)
+// and the reads of x from LDS (208 bytes per unit and token, shared by R rows).
+// 5 tokens: gate and up 2 x 12288 x 4096 Q4_K 44 us where five token steps take 69,
+// 4096 x 12288 39 (47); 6 tokens: a 151936 x 1024 Q8_0 classifier 61 us (6 x 27).
+constexpr int NT_THREADS = 512, NT_NW = NT_THREADS / WAVE, NT_KS = 4096;
+static __host__ __device__ constexpr int nt_stride(int ks) { return 3 * (ks / 16) + ks / 32; }  // 16-byte units per token
+template <int T, int R, int NM, bool NORM>
+__global__ __launch_bounds__(NT_THREADS) void gemv_nt_kernel(GemvNtArgs a) {
+    using W = typename Types<T>::W;
+    using X = typename Types<T>::X;
+    extern __shared__ u32x4 smem[];
+    __shared__ float red[GEMV_NT_MAX][NT_NW];
+    __shared__ float rsc[GEMV_NT_MAX];
+    __shared__ uint32_t tile_ctr;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
+    const int n = a.n, K = a.K, ks = a.ks, ps = nt_stride(ks);
+    int seg = 0;
+    if (NM == 1)
+        for (int i = 1; i < a.nseg; i++)
+            if ((int)blockIdx.x >= a.seg[i].wg_begin) seg = i;
+    const int seg_end = NM == 1 && seg + 1 < a.nseg ? a.seg[seg + 1].wg_begin : a.total_wgs;
+    const int nwg = seg_end - a.seg[seg].wg_begin, w = (int)blockIdx.x - a.seg[seg].wg_begin, ntiles = a.seg[seg].ntiles;
+    const int tb = (int)((long)ntiles * w / nwg), ntl = (int)((long)ntiles * (w + 1) / nwg) - tb;
+    const DMat &m0 = a.seg[seg].m;
+    const DMat &m1 = a.seg[NM == 2 ? 1 : seg].m;
+    const int lpr = a.lpr, grp = lane / lpr, j = lane & (lpr - 1), rpt = WAVE / lpr * R, rows_m = m0.rows;
+    const int wrow0 = tb * rpt, nrow = min((tb + ntl) * rpt, rows_m) - wrow0, rw = a.rows_wg;
+    float *yo = (float *)(smem + (size_t)n * ps);  // [NM][n][rw]
+    auto planes = [&](int t) {
+        u32x4 *b = smem + t * ps;
+        float *f = (float *)(b + 3 * (ks / 16));
+        return XQ{b, b + ks / 16, b + 2 * (ks / 16), f, f + ks / 32, f + ks / 16};
+    };
+    W ring[2][NM][R];
+    for (int k0 = 0; k0 < K; k0 += ks) {
+        const int kl = min(ks, K - k0), u0 = k0 >> 6, U = kl >> 6, ju = min(j, U - 1);
+        auto issue = [&](int t, W (&wv)[NM][R]) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int row = t < ntl ? min((tb + t) * rpt + grp * R + r, rows_m - 1) : 0;
+                wload(m0, row, u0 + ju, wv[0][r]);
+                if (NM == 2) wload(m1, row, u0 + ju, wv[NM - 1][r]);
+            }
+        };
+        // x, then the first weights (loads return in order), then the planes
+        constexpr int XP = NT_KS / 4 / NT_THREADS;  // float4 per thread and token
+        float4 xv[GEMV_NT_MAX][XP], nw[XP];
+#pragma unroll
+        for (int i = 0; i < XP; i++) {
+            const int c = min(tid + i * NT_THREADS, kl / 4 - 1);
+            if (NORM) nw[i] = ((const float4 *)(a.norm_w + k0))[c];
+#pragma unroll
+            for (int t = 0; t < GEMV_NT_MAX; t++)
+                if (t < n) xv[t][i] = ((const float4 *)(a.x + (size_t)t * K + k0))[c];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        int ct = wave;
+        issue(ct, ring[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (k0 > 0) __syncthreads();  // the previous pass has read its planes
+        if (tid == 0) tile_ctr = 0;
+#pragma unroll
+        for (int t = 0; t < GEMV_NT_MAX; t++) {
+            if (t >= n) break;
+            int to = t;
+            asm volatile("" : "+s"(to));  // (the addresses of eight tokens' planes are not kept across passes)
+            const XQ q = planes(to);
+            float ss = 0.f;
+#pragma unroll
+            for (int i = 0; i < XP; i++) {
+                const int c = tid + i * NT_THREADS;  // (kl / 4 is a multiple of 64: whole waves)
+                if (c >= kl / 4) break;
+                float4 v = xv[t][i];
+                if (NORM) {
+                    ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+                    {
+#pragma clang fp contract(off)
+                        v.x = nw[i].x * v.x;
+                        v.y = nw[i].y * v.y;
+                        v.z = nw[i].z * v.z;
+                        v.w = nw[i].w * v.w;
+                    }
+                }
+                quant4(v, c, (uint32_t *)q.hi, (uint32_t *)q.mid, (uint32_t *)q.lo, (float *)q.xs, (float *)q.s32,
+                       (float *)q.s16);
+            }
+            if (NORM) {
+                ss = wave_sum(ss);
+                if (lane == 0) red[t][wave] = k0 > 0 ? red[t][wave] + ss : ss;
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (one token's quantization in registers at a time)
+        }
+        __syncthreads();
+        const bool live = j < U, first = k0 == 0;
+        auto compute = [&](int t, const W (&wv)[NM][R]) {
+            const int lr = t * rpt + grp * R;  // row in the workgroup's range
+#pragma unroll 1
+            for (int tk = 0; tk < n; tk++) {  // one token's slice of x live at a time
+                X xu;
+                xload(planes(tk), ju, xu);
+                float v[NM][R];
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    v[0][r] = wdot(wv[0][r], ju, xu);
+                    if (NM == 2) v[NM - 1][r] = wdot(wv[NM - 1][r], ju, xu);
+                }
+#pragma unroll
+                for (int mi = 0; mi < NM; mi++)
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const float s = lane_group_sum(live ? v[mi][r] : 0.f, lpr);
+                        if (j == 0) {  // (rows past the matrix land in the slack of yo)
+                            float *d = yo + (mi * n + tk) * rw + lr + r;
+                            *d = first ? s : *d + s;
+                        }
+                    }
+            }
+        };
+        auto next = [&]() {
+            uint32_t v = 0;
+            if (lane == 0) v = __hip_atomic_fetch_add(&tile_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            return NT_NW + (int)__builtin_amdgcn_readfirstlane(v);
+        };
+        while (ct < ntl) {
+            int nt = next();
+            issue(nt, ring[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(ct, ring[0]);
+            ct = nt;
+            if (ct >= ntl) break;
+            nt = next();
+            issue(nt, ring[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(ct, ring[1]);
+            ct = nt;
+        }
+    }
+    if (NORM && tid < n) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < NT_NW; i++) s += red[tid][i];
+        rsc[tid] = 1.0f / sqrtf(s / (float)K + a.eps);
+    }
+    __syncthreads();
+    float *y = a.seg[seg].y;
+    for (int t = 0; t < n; t++) {
+        const float sc = NORM ? rsc[t] : 1.f;
+        for (int i = tid; i < nrow; i += NT_THREADS) {
+#pragma clang fp contract(off)
+            float v = yo[t * rw + i] * sc;
+            float *d = y + (size_t)t * rows_m + wrow0 + i;
+            if (NM == 2) {  // infer/forward.odin:128-132
+                v *= 1.0f / (1.0f + expf(-v));
+                v *= yo[(n + t) * rw + i] * sc;
+            }
+            *d = NM == 1 && a.mode == GEMV_ADD ? *d + v : v;
+        }
+    }
+}
+
+bool gemv_nt_supported(const DMat &m) {
+    return (m.type == T_Q4_K || m.type == T_Q6_K || m.type == T_Q8_0) && m.cols % 256 == 0;
+}
+
+template <int T, int R, int NM>
+static const void *gemv_nt_fn(bool norm) {
+    return norm ? (const void *)gemv_nt_kernel<T, R, NM, true> : (const void *)gemv_nt_kernel<T, R, NM, false>;
+}
+template <int T>
+static const void *gemv_nt_fn(int R, int NM, bool norm) {
+    return NM == 2 ? gemv_nt_fn<T, 1, 2>(norm) : R == 2 ? gemv_nt_fn<T, 2, 1>(norm) : gemv_nt_fn<T, 1, 1>(norm);
+}
+
+// Consecutive segments of one type share a launch (a SWIGLU pair is one).  Two rows
+// per lane group (half the x reads) once that still leaves every wave of the GPU a
+// tile; one workgroup per CU, fewer where they would get less than two tiles.
+hipError_t launch_gemv_nt(GemvNtArgs a, hipStream_t st) {
+    const bool sw = a.mode == GEMV_SWIGLU;
+    if (a.n < 1 || a.n > GEMV_NT_MAX || a.nseg < 1 || a.nseg > GEMV_MAX_SEG || a.K <= 0 || a.K % 256 || !a.x ||
+        (sw && (a.nseg != 2 || a.seg[0].m.type != a.seg[1].m.type || a.seg[0].m.rows != a.seg[1].m.rows)))
+        return hipErrorInvalidValue;
+    for (int i = 0; i < a.nseg; i++)
+        if (!gemv_nt_supported(a.seg[i].m) || a.seg[i].m.cols != a.K || (!sw && !a.seg[i].y)) return hipErrorInvalidValue;
+    const int G = device_cus();
+    const int np = (a.K + NT_KS - 1) / NT_KS;  // passes of equal length
+    a.ks = (a.K / 256 + np - 1) / np * 256;
+    a.lpr = 1;
+    while (a.lpr < 64 && a.lpr < a.ks / 64) a.lpr *= 2;
+    for (int i = 0; i < a.nseg;) {
+        int e = i + 1;
+        while (!sw && e < a.nseg && a.seg[e].m.type == a.seg[i].m.type) e++;
+        if (sw) e = 2;
+        GemvNtArgs b = a;
+        b.nseg = e - i;
+        long rows = 0;
+        for (int k = 0; k < b.nseg; k++) {
+            b.seg[k] = a.seg[i + k];
+            if (!sw || k == 0) rows += b.seg[k].m.rows;
+        }
+        const int gpw = WAVE / a.lpr, R = !sw && a.seg[i].m.type != T_Q6_K && rows >= 2L * gpw * G * NT_NW ? 2 : 1;
+        long tiles = 0;
+        const int nd = sw ? 1 : b.nseg;
+        for (int k = 0; k < nd; k++) {
+            b.seg[k].ntiles = (b.seg[k].m.rows + gpw * R - 1) / (gpw * R);
+            tiles += b.seg[k].ntiles;
+        }
+        // (more than one workgroup per CU only where the results would not fit the LDS)
+        size_t lds = 0;
+        for (long cap = G;; cap *= 2) {
+            const int nwg = (int)std::max<long>(nd, std::min<long>(cap, (tiles + 1) / 2));
+            int wg = 0, left = nwg;
+            b.rows_wg = 0;
+            for (int k = 0; k < nd; k++) {
+                int c = k == nd - 1 ? left : (int)std::lround((double)nwg * b.seg[k].ntiles / tiles);
+                c = std::max(1, std::min(c, left - (nd - 1 - k)));
+                b.seg[k].wg_begin = wg;
+                wg += c;
+                left -= c;
+                b.rows_wg = std::max(b.rows_wg, (b.seg[k].ntiles + c - 1) / c * gpw * R);
+            }
+            b.total_wgs = wg;
+            lds = (size_t)a.n * nt_stride(a.ks) * 16 + (size_t)(sw ? 2 : 1) * a.n * b.rows_wg * 4;
+            if (lds <= 156 * 1024 || cap >= tiles) break;
+        }
+        if (lds > 156 * 1024) return hipErrorInvalidValue;
+        const bool norm = a.norm_w != nullptr;
+        const int NM = sw ? 2 : 1;
+        const void *fn = b.seg[0].m.type == T_Q4_K   ? gemv_nt_fn<T_Q4_K>(R, NM, norm)
+                         : b.seg[0].m.type == T_Q6_K ? gemv_nt_fn<T_Q6_K>(R, NM, norm)
+                                                     : gemv_nt_fn<T_Q8_0>(R, NM, norm);
+        void *args[] = {(void *)&b};
+        const hipError_t r = hipLaunchKernel(fn, dim3((unsigned)b.total_wgs), dim3(NT_THREADS), args, lds, st);
+        if (r != hipSuccess) return r;
+        i = e;
+    }
+    return hipGetLastError();
+}
+
 // ------------------------------------ routed experts of a short prefill chunk
 // mt_dot4_kernel: the token loop's int8 dot4 arithmetic over the few pairs
 // (<= MT_MFMA_FEW) of one expert slice.  An item is (expert, pair slice, one

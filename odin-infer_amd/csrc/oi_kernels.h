@@ -200,6 +200,30 @@ enum { MOE_ROWS = 1, MOE_COLS = 2, MOE_ROWS_R = 3 };
 bool gemv_q_moe_supported(const GemvArgs &a, int moe);
 hipError_t launch_gemv_q_moe(const GemvArgs &a, int moe, hipStream_t st);
 
+// gemv.hip: the token step's GEMV for n <= GEMV_NT_MAX tokens at once, each weight
+// read and unpacked once for all of them (the prompt's trailing tokens and short
+// drafts, every position's classifier): y[t][r] = W[r] . x[t] in the token
+// step's arithmetic.  x [n][K], y [n][rows] f32.
+constexpr int GEMV_NT_MAX = 8;
+struct GemvNtSeg {
+    DMat m;
+    float *y;
+    int32_t wg_begin, ntiles;
+};
+struct GemvNtArgs {
+    GemvNtSeg seg[GEMV_MAX_SEG];
+    int32_t nseg, mode;          // GEMV_STORE, GEMV_ADD (into y) or GEMV_SWIGLU (seg[0] gate, seg[1] up, y of seg[0])
+    int32_t n, K;
+    const float *x;
+    const float *norm_w;         // if set: x is replaced by rmsnorm(x) * norm_w
+    float eps;
+    // the plan (plan_gemv_nt): columns per pass, lanes per row, workgroups, rows of the largest workgroup
+    int32_t ks, lpr, total_wgs, rows_wg;
+};
+// whether the kernel takes the matrices (one type and row length)
+bool gemv_nt_supported(const DMat &m);
+hipError_t launch_gemv_nt(GemvNtArgs a, hipStream_t st);
+
 // gemm.hip: batched projection c[t][r] = sum_k f16(deq(W))[r][k] x[t][k]
 bool gemm_supported(const DMat &m);
 // K slices for n tokens when part_bytes of partial products fit (1 = none)
@@ -238,9 +262,10 @@ hipError_t launch_pf_qkv(const PfQkvArgs &a, int head_dim, hipStream_t st);
 // sigmoid before rounding (the Qwen3.5 attention's output gate)
 // ws: optional scratch for the key-split form of short chunks (head_dim 256:
 // [splits][T][n_heads][head_dim + 2] floats, splits <= 16); unused if too small
+// out: f16 rows, or with out32 set f32 rows there instead
 hipError_t launch_pf_attn(const float *q, const uint16_t *kc, const uint16_t *vc, uint16_t *out, int T, int pos0,
                           int seq_len, int n_heads, int n_kv_heads, int head_dim, hipStream_t st,
-                          const float *gate = nullptr, float *ws = nullptr, size_t ws_bytes = 0);
+                          const float *gate = nullptr, float *ws = nullptr, size_t ws_bytes = 0, float *out32 = nullptr);
 hipError_t launch_pf_add(float *x, const float *part, int split, int64_t total, hipStream_t st);
 // x += partial-product sums (part may be null), then out = f16(rmsnorm(x) * w); dim <= 16384
 // out32: null, or [T][dim] f32 that receives the norm's f32 result as well

@@ -212,12 +212,18 @@ struct PfAttnArgs {
     uint16_t *out;              // [T][n_heads * head_dim] f16 (the wo projection's input)
     int32_t pos0, seq_len, n_heads, n_kv_heads;
     const float *gate;          // null, or [T][n_heads * head_dim]: out *= sigmoid(gate) (Qwen3.5)
+    float *out32;               // null, or f32 rows in place of out's
 };
 
 // the attention output of one element, gated when the layer has a gate
 static __device__ __forceinline__ float pf_gated(const PfAttnArgs &a, float o, size_t i) {
 #pragma clang fp contract(off)
     return a.gate ? o * sigmoid_ref(a.gate[i]) : o;
+}
+static __device__ __forceinline__ void pf_put(const PfAttnArgs &a, float o, size_t i) {
+    const float v = pf_gated(a, o, i);
+    if (a.out32) a.out32[i] = v;
+    else a.out[i] = f2h(v);
 }
 
 // Causal attention of token t (query head h, grid (n_heads, T)) over positions
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(WG) void pf_attn_kernel(PfAttnArgs a) {
         float acc = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; w++) acc += ow[w][i] * sc[w];
-        a.out[(size_t)t * QD + h * HD + i] = f2h(pf_gated(a, acc / lt, (size_t)t * QD + h * HD + i));
+        pf_put(a, acc / lt, (size_t)t * QD + h * HD + i);
     }
 }
 
@@ -497,6 +503,10 @@ __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float
             float r[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) r[e] = pf_gated(a, o[dt][e] / lsum, d0 + 16 * dt + e);
+            if (a.out32) {
+                *(float4 *)(a.out32 + d0 + 16 * dt) = make_float4(r[0], r[1], r[2], r[3]);
+                continue;
+            }
             const uint32_t w0 = (uint32_t)f2h(r[0]) | ((uint32_t)f2h(r[1]) << 16);
             const uint32_t w1 = (uint32_t)f2h(r[2]) | ((uint32_t)f2h(r[3]) << 16);
             *(u32x2 *)(dst + 16 * dt) = u32x2{w0, w1};
@@ -542,7 +552,7 @@ __global__ __launch_bounds__(WG) void pf_fattn_merge_kernel(PfAttnArgs a, int T,
 #pragma unroll
     for (int e = 0; e < DPL; e++) {
         const size_t i = (size_t)p * HD + lane + WAVE * e;
-        a.out[i] = f2h(pf_gated(a, O[e] / L, i));
+        pf_put(a, O[e] / L, i);
     }
 }
 
@@ -584,8 +594,8 @@ hipError_t launch_pf_qkv(const PfQkvArgs &a, int head_dim, hipStream_t st) {
 
 hipError_t launch_pf_attn(const float *q, const uint16_t *kc, const uint16_t *vc, uint16_t *out, int T, int pos0,
                           int seq_len, int n_heads, int n_kv_heads, int head_dim, hipStream_t st, const float *gate,
-                          float *ws, size_t ws_bytes) {
-    PfAttnArgs a{q, kc, vc, out, pos0, seq_len, n_heads, n_kv_heads, gate};
+                          float *ws, size_t ws_bytes, float *out32) {
+    PfAttnArgs a{q, kc, vc, out, pos0, seq_len, n_heads, n_kv_heads, gate, out32};
     const dim3 grid((unsigned)n_heads, (unsigned)T);
     const dim3 fgrid((unsigned)n_heads, (unsigned)((T + 63) / 64));
     // The key blocks of a query tile are split over workgroups where the tiles

@@ -467,3 +467,29 @@ def test_verify_batch_vs_oracle(make_model, name, seed):
         infer.engine_destroy(e)
         infer.engine_destroy(e2)
         r.close()
+
+
+@pytest.mark.parametrize("name", ["tiny-q4_k", "tiny-q8_0", "moe-tiny", "qwen35-tiny", "qwen35-moe-tiny", "8b-1layer-q4_k"])
+@pytest.mark.parametrize("n", [2, 3, 5, 7])
+def test_few_tokens_equal_the_token_step(make_model, name, n):
+    """2-7 tokens in one pass (every row's logits) against the same tokens through
+    the token step on a second engine: the same arithmetic in another order (the
+    8B shape's 12288-column rows run in three passes), so the rows differ by f32
+    rounding and by the f16 cache values that it tips over: 2^-11 of a few cached
+    values of a few hundred, below 5e-4 of the largest logit.  The states after
+    are the same to that measure, and a row is the same in a shorter call."""
+    path = make_model(name)
+    opts = infer.Engine_Opts(max_ctx=128)
+    (e, _), (s, _) = infer.engine_load(path, opts), infer.engine_load(path, opts)
+    try:
+        t = _tokens(n + 1, 24 + n, e.config.vocab_size)
+        for x in (e, s):
+            infer.engine_forward_batch(x, t[:24], 0)
+        rows = infer.engine_verify_batch(e, t[24:], 24).copy()
+        ref = np.array([infer.engine_forward(s, int(t[24 + i]), 24 + i).copy() for i in range(n)])
+        errs = [scaled_err(rows[i], ref[i]) for i in range(n)]
+        assert max(errs) <= 5e-4, errs
+        assert scaled_err(infer.engine_forward(e, 5, 24 + n), infer.engine_forward(s, 5, 24 + n)) <= 5e-4
+    finally:
+        infer.engine_destroy(e)
+        infer.engine_destroy(s)
