@@ -1589,8 +1589,12 @@ __global__ __launch_bounds__(NWV * WAVE) void mt_q4i8_kernel(MtGemvArgs a) {
     static_assert(SBS == 1 || SBS == 2, "one or two super-blocks per step");
     static_assert(HT == 0 || ((4 * SBS) % HT == 0 && HT % 2 == 0), "a step's headers in fixed registers");
     const bool second = a.mat_items > 0 && (int)blockIdx.x >= a.mat_items;
-    const int it = second ? (int)blockIdx.x - a.mat_items : (int)blockIdx.x;
-    if (it >= *a.nitems) return;
+    // consecutive blocks go to different XCDs: each XCD takes a contiguous range of
+    // the items, so the pair slices of one expert read its rows from one L2 (504
+    // tokens of config 5, three slices an expert: gate/up 297 -> 290 us, down 180 -> 178)
+    const int bid = second ? (int)blockIdx.x - a.mat_items : (int)blockIdx.x, nit = *a.nitems, per = (nit + 7) >> 3;
+    const int it = (bid & 7) * per + (bid >> 3);
+    if ((bid >> 3) >= per || it >= nit) return;
     const int K = a.K, U = K >> 6, NSB = K >> 8, NSS = NSB / SBS;  // NSB % SBS == 0
     const int e = a.items[2 * it], slice = a.items[2 * it + 1] >> 16, tile = a.items[2 * it + 1] & 0xFFFF;
     const int base = a.off[e] + slice * NP, n = min(NP, a.cnt[e] - slice * NP);
@@ -1900,6 +1904,7 @@ hipError_t launch_mt_q4i8(const MtGemvArgs &a, int max_items, hipStream_t st) {
         a.pair_slice != MT_MFMA_FEW || a.xdiv <= 0 || max_items <= 0 || a.dense_n > 0)
         return hipErrorInvalidValue;
     MtGemvArgs b = a;
+    max_items = (max_items + 7) & ~7;  // (the kernel deals the items out in eight ranges)
     b.mat_items = a.swiglu ? max_items : 0;  // gate into y, up into y2 (the SwiGLU is the consumer's)
     const size_t lds = mt_q4i8_lds(a.K, QI_NW);
     const dim3 grid((unsigned)(a.swiglu ? 2 * max_items : max_items)), block(QI_NW * WAVE);

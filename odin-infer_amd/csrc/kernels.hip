@@ -1446,42 +1446,67 @@ __device__ __forceinline__ int block_excl_scan(int v, int *wsum, int *total) {
 // row tile) of the gate/up and down multi-token GEMVs: tiles_gu / tiles_dn
 // row tiles per slice of pair_slice pairs of each chosen expert.
 __global__ __launch_bounds__(1024) void pf_moe_group_kernel(PfMoeArgs a) {
-    __shared__ int cnt[1024], fill[1024], wsum[16];
-    const int ne = a.n_experts + (a.kp > a.top_k ? 1 : 0), P = a.T * a.kp, e = threadIdx.x;
+    __shared__ int cnt[1024], fill[1024], sl[1025], wsum[16];
+    const bool shared = a.kp > a.top_k;  // slot top_k of every token is the shared expert, expert n_experts
+    const int ne = a.n_experts + (shared ? 1 : 0), P = a.T * a.kp, e = threadIdx.x;
     if (e < ne) {
-        cnt[e] = 0;
+        cnt[e] = shared && e == a.n_experts ? a.T : 0;
         fill[e] = 0;
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) atomicAdd(&cnt[min(max(a.ids[p], 0), ne - 1)], 1);
+    constexpr int NB = 6;  // pairs per thread in flight
+    auto pairs = [&](auto &&f) {
+        for (int p0 = threadIdx.x; p0 < P; p0 += NB * (int)blockDim.x) {
+            int id[NB];
+#pragma unroll
+            for (int i = 0; i < NB; i++) id[i] = a.ids[min(p0 + i * (int)blockDim.x, P - 1)];
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                const int p = p0 + i * (int)blockDim.x;
+                if (p < P) f(p, min(max(id[i], 0), ne - 1));
+            }
+        }
+    };
+    // (the shared expert's pairs are known: no counting, no contended slot)
+    pairs([&](int p, int x) {
+        if (!(shared && p % a.kp == a.top_k)) atomicAdd(&cnt[x], 1);
+    });
     __syncthreads();
     const int c = e < ne ? cnt[e] : 0, ns = (c + a.pair_slice - 1) / a.pair_slice;
-    int tp, tg, td;
+    int tp, ts;
     const int off = block_excl_scan(c, wsum, &tp);
-    const int og = block_excl_scan(ns * a.tiles_gu, wsum, &tg);
-    const int od = block_excl_scan(ns * a.tiles_dn, wsum, &td);
+    const int os = block_excl_scan(ns, wsum, &ts);  // pair slices before expert e
     if (e < ne) {
         a.off[e] = off;
         a.cnt[e] = c;
-        for (int i = 0; i < ns * a.tiles_gu; i++) {
-            a.items_gu[2 * (og + i)] = e;
-            a.items_gu[2 * (og + i) + 1] = ((i / a.tiles_gu) << 16) | (i % a.tiles_gu);
-        }
-        for (int i = 0; i < ns * a.tiles_dn; i++) {
-            a.items_dn[2 * (od + i)] = e;
-            a.items_dn[2 * (od + i) + 1] = ((i / a.tiles_dn) << 16) | (i % a.tiles_dn);
-        }
         fill[e] = off;  // the next free slot of e
     }
-    if (threadIdx.x == 0) {
-        a.nitems[0] = tg;
-        a.nitems[1] = td;
+    sl[e] = os;
+    if (e == 0) {
+        sl[1024] = ts;
+        a.nitems[0] = ts * a.tiles_gu;
+        a.nitems[1] = ts * a.tiles_dn;
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
-        const int x = min(max(a.ids[p], 0), ne - 1);
-        a.list[atomicAdd(&fill[x], 1)] = p;
+    // work items, a thread per pair slice (an expert of many slices written by its
+    // own thread alone took most of the kernel: the shared expert has T / pair_slice)
+    for (int i = threadIdx.x; i < ts; i += blockDim.x) {
+        int lo = 0, hi = ne - 1;  // the last expert with sl <= i
+        while (lo < hi) {
+            const int m = (lo + hi + 1) >> 1;
+            if (sl[m] <= i) lo = m;
+            else hi = m - 1;
+        }
+        const int s = i - sl[lo];
+        for (int t = 0; t < a.tiles_gu; t++)
+            *(int2 *)(a.items_gu + 2 * (i * a.tiles_gu + t)) = make_int2(lo, (s << 16) | t);
+        for (int t = 0; t < a.tiles_dn; t++)
+            *(int2 *)(a.items_dn + 2 * (i * a.tiles_dn + t)) = make_int2(lo, (s << 16) | t);
     }
+    pairs([&](int p, int x) {
+        if (shared && p % a.kp == a.top_k) a.list[fill[a.n_experts] + p / a.kp] = p;
+        else a.list[atomicAdd(&fill[x], 1)] = p;
+    });
 }
 
 // out[t][r] = sum over the token's slots s (rank order, the shared expert
