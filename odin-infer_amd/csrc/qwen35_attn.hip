@@ -377,16 +377,18 @@ __global__ __launch_bounds__(q35_lane_threads(G)) void q35_lane_kernel(Q35Args a
 }
 
 // Merge of a head's splits: one query head and 64 of its dimensions per
-// workgroup (grid (n_heads, HD / 64)), the 4 waves taking every 4th split,
-// the first Q35_PF splits' values requested together with the (m, l) pairs
-// (one memory round trip); the split weights exp(m_s - M) are formed once in
-// LDS by one wave.  out = (o / l) sigmoid(gate).
-constexpr int Q35_PF = 20;
+// workgroup (grid (n_heads, HD / 64)), wave w taking splits w, w + Q35_CW, ...,
+// the first Q35_PF of each requested together with the (m, l) pairs (one memory
+// round trip, up to Q35_CW * Q35_PF = 128 splits); the split weights exp(m_s - M)
+// are formed once in LDS by one wave.  out = (o / l) sigmoid(gate).  Bound by
+// those round trips, 64 workgroups of a few KB each: with 4 waves and 20 values
+// in flight 128 splits took a chain of 12 further loads, 7.0 us against 3.7.
+constexpr int Q35_CW = 16, Q35_PF = 8;  // waves; splits per wave in the first round trip
 template <int HD>
-__global__ __launch_bounds__(WG) void q35_combine_kernel(Q35Args a) {
+__global__ __launch_bounds__(Q35_CW * WAVE) void q35_combine_kernel(Q35Args a) {
 #pragma clang fp contract(off)
     __shared__ float wm[Q35_MAXS], wl[Q35_MAXS];
-    __shared__ float ored[WG / WAVE][WAVE];
+    __shared__ float ored[Q35_CW][WAVE];
     __shared__ float Ls;
     const int pos = a.state ? a.state[ST_POS] : a.pos;
     const int h = blockIdx.x, ns = (pos + Q35_CH) / Q35_CH, t = threadIdx.x;
@@ -395,11 +397,11 @@ __global__ __launch_bounds__(WG) void q35_combine_kernel(Q35Args a) {
     float ov[Q35_PF];
 #pragma unroll
     for (int k = 0; k < Q35_PF; k++) {
-        const int s = wave + (WG / WAVE) * k;
+        const int s = wave + Q35_CW * k;
         ov[k] = s < ns ? pb[(size_t)s * (HD + 2) + i] : 0.f;
     }
     const float gate = a.qproj[(size_t)h * 2 * HD + HD + i];
-    for (int s = t; s < ns; s += WG) {
+    for (int s = t; s < ns; s += Q35_CW * WAVE) {
         wm[s] = pb[(size_t)s * (HD + 2) + HD];
         wl[s] = pb[(size_t)s * (HD + 2) + HD + 1];
     }
@@ -422,15 +424,23 @@ __global__ __launch_bounds__(WG) void q35_combine_kernel(Q35Args a) {
     float O = 0.f;
 #pragma unroll
     for (int k = 0; k < Q35_PF; k++) {
-        const int s = wave + (WG / WAVE) * k;
+        const int s = wave + Q35_CW * k;
         if (s < ns) O += ov[k] * wm[s];
     }
-    for (int s = wave + (WG / WAVE) * Q35_PF; s < ns; s += WG / WAVE) O += pb[(size_t)s * (HD + 2) + i] * wm[s];
+#pragma unroll 8
+    for (int s = wave + Q35_CW * Q35_PF; s < ns; s += Q35_CW) O += pb[(size_t)s * (HD + 2) + i] * wm[s];
     ored[wave][lane] = O;
     __syncthreads();
-    if (wave == 0)
-        a.out[(size_t)h * HD + i] = (((ored[0][lane] + ored[1][lane]) + (ored[2][lane] + ored[3][lane])) / Ls) *
-                                   sigmoid_ref(gate);
+    if (wave == 0) {
+        float v[Q35_CW];
+#pragma unroll
+        for (int w = 0; w < Q35_CW; w++) v[w] = ored[w][lane];
+#pragma unroll
+        for (int w = Q35_CW / 2; w >= 1; w >>= 1)
+#pragma unroll
+            for (int k = 0; k < w; k++) v[k] = v[2 * k] + v[2 * k + 1];
+        a.out[(size_t)h * HD + i] = (v[0] / Ls) * sigmoid_ref(gate);
+    }
 }
 
 int q35_max_splits(int seq_len) { return (seq_len + Q35_CH - 1) / Q35_CH; }
@@ -458,13 +468,13 @@ hipError_t launch_q35_attn(const Q35Args &a, int head_dim, hipStream_t st) {
             case 4: hipLaunchKernelGGL((q35_lane_kernel<HD, 4>), gl, dim3(q35_lane_threads(4)), 0, st, a); break;
             default: hipLaunchKernelGGL((q35_lane_kernel<HD, 8>), gl, dim3(q35_lane_threads(8)), 0, st, a); break;
             }
-            hipLaunchKernelGGL(q35_combine_kernel<HD>, g3, dim3(WG), 0, st, a);
+            hipLaunchKernelGGL(q35_combine_kernel<HD>, g3, dim3(Q35_CW * WAVE), 0, st, a);
             return;
         }
         if (gw == 4) hipLaunchKernelGGL((q35_attn_kernel<HD, 4>), g2, dim3(WG), 0, st, a);
         else if (gw == 2) hipLaunchKernelGGL((q35_attn_kernel<HD, 2>), g2, dim3(WG), 0, st, a);
         else hipLaunchKernelGGL((q35_attn_kernel<HD, 1>), g2, dim3(WG), 0, st, a);
-        hipLaunchKernelGGL(q35_combine_kernel<HD>, g3, dim3(WG), 0, st, a);
+        hipLaunchKernelGGL(q35_combine_kernel<HD>, g3, dim3(Q35_CW * WAVE), 0, st, a);
     };
     if (head_dim == 256) attn(std::integral_constant<int, 256>{});
     else if (head_dim == 128) attn(std::integral_constant<int, 128>{});

@@ -51,6 +51,22 @@ def test_qwen35_attn_vs_oracle(monkeypatch, kernel, n_heads, n_kv, hd, rd, seq_l
     assert dk.max() <= 1  # k after norm and RoPE: at most one f16 ulp apart
 
 
+@pytest.mark.parametrize("kernel,pos0", [("lanes", 8190), ("groups", 8190), ("lanes", 12345)])
+def test_qwen35_merge_past_its_first_round_trip(monkeypatch, kernel, pos0):
+    """Positions on both sides of 8192, where the merge's waves take splits past
+    the 128 that they request together (128 -> 129 splits), and 193 splits.  The
+    scores and the merge are f32 sums of at most 12,348 terms, each rounded to
+    2^-24 of partial sums no larger than the result's own scale: 1e-4 as above."""
+    monkeypatch.setenv("OI_Q35_ATTN", kernel)
+    T, seq_len = 4, pos0 + 8
+    qproj, k, v, qn, kn, kc, vc = _case(np.random.default_rng(pos0), 8, 1, 128, seq_len, pos0, T)
+    args = (8, 1, 128, 64, seq_len, 1e-6, pos0, qproj, k, v, qn, kn, refcpu.inv_freq(1e7, 64), kc, vc)
+    out, gkc, gvc = qwen35.attn_steps(*args)
+    rout, rkc, rvc = refcpu.qwen35_attn_steps(*args)
+    assert np.max(np.abs(np.float64(out) - rout)) / np.max(np.abs(rout)) <= 1e-4
+    assert np.array_equal(gvc, rvc)
+
+
 def test_qwen35_attn_rejects():
     qproj, k, v, qn, kn, kc, vc = _case(np.random.default_rng(1), 4, 2, 96, 64, 0, 1)
     with pytest.raises(_native.OIError):  # head_dim 96 is not built
