@@ -535,25 +535,31 @@ static int normalize_split(int nchunk, int split) {
 }
 
 // Token tiles (of 16) per workgroup and K split of a launch of `rt` row tiles: the
-// pair of least estimated time with at most `cap` slices.  Estimated (us, measured
-// on 4096 x n x 4096 / 12288 with every CU busy): a chunk at 128 tokens 2.2, 64
-// tokens 1.6, 32 tokens 0.9; a workgroup's fixed time; rounds of one workgroup per
-// CU; the further slices written and read back; the reduction's launch if the
-// caller has one.
+// pair of least estimated time with at most `cap` slices.  The estimate (us) has a
+// CU's workgroups one after another (two of 32 tokens fit a CU, and take twice as
+// long): a chunk and a fixed time per workgroup, every slice written and read back,
+// and the reduction's launch if the caller has one.  Its constants are fitted to
+// 220 shapes (500 - 12288 rows, 1024 - 12288 columns, 8 - 512 tokens, the three
+// types) run at every tile and 11 splits: the chosen pair takes 1.2% (Q4_K), 0.4%
+// (Q6_K) and 0.3% (Q8_0) longer than the fastest one on average.  With the tile
+// taken from n alone (32 tokens up to 32, 64 or 128 above) and the constants of
+// two large matrices it was 4.1, 3.0 and 2.6%, and up to 41%: few rows or columns
+// want more and smaller tiles at any n (3095 x 1024 Q4_K, 157 tokens: 9.1 us at 32
+// tokens a tile, 10.6 at 64, 12.2 at 64 with 16-row waves).
 struct GemmPlan {
     int tt, split;
 };
 static GemmPlan gemm_plan(int type, int rt, int nchunk, int32_t n, double out, int cap, bool reduce) {
-    GemmPlan best{0, 1};
+    GemmPlan best{2, 1};
     double bt = 1e30;
-    const int tmax = n <= 32 ? 2 : n <= 64 || type == T_Q8_0 ? 4 : 8;
-    for (int tt = n <= 32 ? 2 : 4; tt <= tmax; tt *= 2) {
-        const double chunk = tt == 8 ? 2.2 : tt == 4 ? 1.6 : 0.9, fixed = tt == 8 ? 5.0 : 4.0;
+    const double unit = type == T_Q4_K ? 0.9 : 1.0;  // (the fewest instructions per weight)
+    for (int tt = 2; tt <= (type == T_Q8_0 ? 4 : 8); tt *= 2) {
+        const double chunk = unit * (tt == 8 ? 1.9 : tt == 4 ? 1.65 : 1.35), fixed = tt == 8 ? 6.3 : tt == 4 ? 2.9 : 2.2;
         const int tiles = rt * ((n + 16 * tt - 1) / (16 * tt));
         for (int s = 1; s <= std::max(1, nchunk / 2) && s <= cap; s++) {
             if (normalize_split(nchunk, s) != s) continue;
             const double t = (tiles * s + 255) / 256 * (((nchunk + s - 1) / s) * chunk + fixed) +
-                             (s > 1 ? (s - 1) * out * 8.0 / 8e6 + (reduce ? 4.0 : 0.0) : 0.0);
+                             (s > 1 ? s * out * 1.4e-6 + (reduce ? 3.3 : 0.0) : 0.0);
             if (t < bt) {
                 bt = t;
                 best = GemmPlan{tt, s};
