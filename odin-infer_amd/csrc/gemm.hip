@@ -7,7 +7,7 @@
 // reference harness's B[K][N] and C[M][N]; same products).
 //
 // Work layout: a workgroup of 8 waves computes 128 rows x 16 TT tokens (TT = 8,
-// 4 or 2) over a slice of K, walked in chunks of 256 (one Q4_K / Q6_K
+// 6, 4 or 2) over a slice of K, walked in chunks of 256 (one Q4_K / Q6_K
 // super-block, eight Q8_0 blocks).  Per chunk the activations and the raw
 // weight bytes are staged in LDS; wave (rg, kh) takes rows 32 rg .. +31 and
 // half kh of the chunk's sixteen 16-wide K steps, in v_mfma_f32_32x32x16_f16
@@ -240,10 +240,11 @@ struct GQ6K {
 
 // Q8_0, chunk = blocks 8c .. 8c+7; unit u of it: blocks 8c + 2u and 8c + 2u + 1;
 // plane 2 blk + half holds bytes 16 half .. +15 of block blk.  Step st = 4 blk + 2
-// half + b: weight 64u + 8st + e, octet 8u + st; K half kh: block kh of the unit.  (Four planes beside 128 tokens would not fit the LDS:
-// TMAX 4.)  ggml/quant.odin:87-96.
+// half + b: weight 64u + 8st + e, octet 8u + st; K half kh: block kh of the unit.  (Four planes
+// and the scales beside 128 tokens would be 2 KB more than the LDS: TMAX 6, 96
+// tokens.)  ggml/quant.odin:87-96.
 struct GQ80 {
-    static constexpr int PL = 4, TMAX = 4;
+    static constexpr int PL = 4, TMAX = 6;
     static constexpr bool D = false;
     static __device__ __forceinline__ const u32x4 *tail_of(const DMat &m, int row) {  // eight block scales per chunk
         return (const u32x4 *)m.d + (size_t)row * (m.cols >> 8);
@@ -483,20 +484,22 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q_kernel(GemmArgs a) {
         }
     } else {
         float *out = g.c + (size_t)bz * a.n * M;
+        if (M & 3) {  // rows of C not 16-byte aligned: one float per lane, side by side
+            const float *yf = (const float *)yo;
+            const int row = tid & (GM_ROWS - 1), r0 = bx * GM_ROWS + row;
+#pragma unroll 8
+            for (int tk = tid / GM_ROWS; tk < TOK; tk += GM_THREADS / GM_ROWS) {
+                const int k = 4 * (tk * 32 + ((row >> 2) ^ (tk & 7))) + (row & 3);
+                if (t0 + tk < a.n && r0 < M) out[(size_t)(t0 + tk) * M + r0] = yf[k] + yf[4 * TOK * 32 + k];
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < XPT; i++) {
             const int p = tid + i * GM_THREADS, tk = p >> 5, cc = p & 31;
             if (t0 + tk >= a.n) continue;
-            const f32x4v v = sum(tk, cc);
             const int r0 = bx * GM_ROWS + 4 * cc;
-            float *dst = out + (size_t)(t0 + tk) * M + r0;
-            if (r0 + 3 < M && (M & 3) == 0) {
-                *(f32x4v *)dst = v;
-                continue;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (r0 + e < M) dst[e] = v[e];
+            if (r0 < M) *(f32x4v *)(out + (size_t)(t0 + tk) * M + r0) = sum(tk, cc);
         }
     }
 }
@@ -539,13 +542,14 @@ static int normalize_split(int nchunk, int split) {
 // CU's workgroups one after another (two of 32 tokens fit a CU, and take twice as
 // long): a chunk and a fixed time per workgroup, every slice written and read back,
 // and the reduction's launch if the caller has one.  Its constants are fitted to
-// 220 shapes (500 - 12288 rows, 1024 - 12288 columns, 8 - 512 tokens, the three
-// types) run at every tile and 11 splits: the chosen pair takes 1.2% (Q4_K), 0.4%
-// (Q6_K) and 0.3% (Q8_0) longer than the fastest one on average.  With the tile
+// 240 shapes (500 - 12288 rows, 1024 - 12288 columns, 8 - 512 tokens, the three
+// types) run at every tile and 11 splits: the chosen pair takes 1.4% (Q4_K), 0.4%
+// (Q6_K) and 0.2% (Q8_0) longer than the fastest one on average.  With the tile
 // taken from n alone (32 tokens up to 32, 64 or 128 above) and the constants of
 // two large matrices it was 4.1, 3.0 and 2.6%, and up to 41%: few rows or columns
 // want more and smaller tiles at any n (3095 x 1024 Q4_K, 157 tokens: 9.1 us at 32
-// tokens a tile, 10.6 at 64, 12.2 at 64 with 16-row waves).
+// tokens a tile, 10.6 at 64).  Tiles of 96 tokens are worth 3.5% on average for
+// Q8_0, which has no larger one, and 0.7% for the others.
 struct GemmPlan {
     int tt, split;
 };
@@ -553,8 +557,10 @@ static GemmPlan gemm_plan(int type, int rt, int nchunk, int32_t n, double out, i
     GemmPlan best{2, 1};
     double bt = 1e30;
     const double unit = type == T_Q4_K ? 0.9 : 1.0;  // (the fewest instructions per weight)
-    for (int tt = 2; tt <= (type == T_Q8_0 ? 4 : 8); tt *= 2) {
-        const double chunk = unit * (tt == 8 ? 1.9 : tt == 4 ? 1.65 : 1.35), fixed = tt == 8 ? 6.3 : tt == 4 ? 2.9 : 2.2;
+    for (int tt : {2, 4, 6, 8}) {
+        if (tt == 8 && type == T_Q8_0) continue;
+        const double chunk = unit * (tt == 8 ? 1.9 : tt == 6 ? 1.78 : tt == 4 ? 1.65 : 1.35);
+        const double fixed = tt == 8 ? 6.3 : tt == 6 ? 4.5 : tt == 4 ? 2.9 : 2.2;
         const int tiles = rt * ((n + 16 * tt - 1) / (16 * tt));
         for (int s = 1; s <= std::max(1, nchunk / 2) && s <= cap; s++) {
             if (normalize_split(nchunk, s) != s) continue;
@@ -584,6 +590,7 @@ static hipError_t gemm_launch_t(const GemmArgs &a, int blocks, int tt, hipStream
     switch (tt) {
     case 2: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 2>), grid, block, gm_lds<G>(2), st, a); break;
     case 4: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 4>), grid, block, gm_lds<G>(4), st, a); break;
+    case 6: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 6>), grid, block, gm_lds<G>(6), st, a); break;
     default:
         if constexpr (G::TMAX >= 8) hipLaunchKernelGGL((gemm_q_kernel<G, NP, 8>), grid, block, gm_lds<G>(8), st, a);
         else return hipErrorInvalidValue;

@@ -187,3 +187,21 @@ def test_gemm_tile_edges(kind, m, n, k):
     x = x16(rng.uniform(-1, 1, size=(n, k)))
     err = scaled_err(ggml.gemm(kind, w, m, k, x), refcpu.gemm_f16(w, kind, m, k, x))
     assert err <= k ** 1.5 * 2.0 ** -24, "%d %dx%dx%d scaled error %.3g" % (kind, m, n, k, err)
+
+
+@pytest.mark.parametrize("kind,m,n,k", [(8, 12288, 96, 4096), (8, 12289, 97, 1024), (8, 1537, 191, 256),
+                                        (14, 4097, 192, 512), (12, 511, 95, 2048)])
+def test_gemm_96_token_tiles_and_odd_rows(kind, m, n, k):
+    """Sizes about multiples of 96 tokens, where that tile is chosen or just not, and
+    row counts whose results are stored a float per lane (not a multiple of 4);
+    the bound is test_gemm_tile_edges'.  The oracle takes the first and last tile's rows."""
+    rng = np.random.default_rng(m + n + k + kind)
+    w = gemm_blocks(kind, m, k, rng)
+    x = x16(rng.uniform(-1, 1, size=(n, k)))
+    y = ggml.gemm(kind, w, m, k, x)
+    rb = np.asarray(w).reshape(m, -1)
+    for r in (slice(0, 130), slice(max(0, m - 130), m)):
+        part = np.ascontiguousarray(rb[r])
+        rows = part.shape[0]
+        err = scaled_err(np.ascontiguousarray(y[:, r]), refcpu.gemm_f16(part.reshape(-1), kind, rows, k, x))
+        assert err <= k ** 1.5 * 2.0 ** -24, "%d %dx%dx%d scaled error %.3g" % (kind, m, n, k, err)
