@@ -1650,6 +1650,16 @@ int prefill_few(oi_engine *e, const int32_t *tokens, int T, int pos, float *rows
 
 namespace {
 
+// The fewest trailing tokens of a call that prefill_few takes (8: none, each goes
+// through the token step).  The DeltaNet kernels need a whole conv window; the
+// SwiGLU pair of launch_gemv_nt is of one type, so a file whose gate and up
+// projections differ in type keeps the token step, which takes any pair.
+int prefill_few_min(const oi_engine *e) {
+    for (const LayerDev &L : e->layers)
+        if (!L.moe && L.w1.type != L.w3.type) return 8;
+    return e->lin_nv > 0 ? std::max(2, (int)e->lin_kernel - 1) : 2;
+}
+
 // engine_forward_batch over tokens[0, n) at pos0 (chunks of a multiple of 8
 // up to PF_MAX_T batched, the trailing 1-7 in the decode path's arithmetic).  rows ==
 // nullptr: the last token's logits in e->logits; otherwise every token's
@@ -1667,6 +1677,7 @@ int prefill_run(oi_engine *e, const int32_t *tokens, int32_t n, int32_t pos0, fl
                                         " out of range (vocab=" + std::to_string(e->cfg.vocab_size) + ")");
     if (hipSetDevice(e->device) != hipSuccess) return fail(OI_E_DEVICE, "hipSetDevice failed");
     const bool batched = prefill_batched_ok(e);
+    const int few_min = prefill_few_min(e);
     if (batched && prefill_alloc(e)) return -1;
     if (ensure_graph(e)) return -1;
     const size_t V = (size_t)e->cfg.vocab_size;
@@ -1678,7 +1689,7 @@ int prefill_run(oi_engine *e, const int32_t *tokens, int32_t n, int32_t pos0, fl
             chunk -= chunk % 8;
             if (prefill_chunk(e, tokens + i, chunk, pos0 + i, rows ? rows + (size_t)i * V : nullptr)) return -1;
             i += chunk;
-        } else if (batched && rem >= (e->lin_nv > 0 ? (int)e->lin_kernel - 1 : 2)) {  // the trailing tokens at once
+        } else if (batched && rem >= few_min) {  // the trailing tokens at once
             if (prefill_few(e, tokens + i, rem, pos0 + i, rows ? rows + (size_t)i * V : nullptr)) return -1;
             i += rem;
         } else {  // one token through the decode path

@@ -156,3 +156,31 @@ def gguf_tensor_data(data):
             out[t] = (start + int.from_bytes(data[off:off + 8], "little"),
                       int.from_bytes(data[off - 4:off], "little"))
     return out
+
+
+def gguf_retype(src, dst, kinds):
+    """Copy the GGUF file `src` to `dst` with some 2-D tensors in another type:
+    kinds = {ending of the tensor name: GGML type}, the values requantized."""
+    import refcpu
+    from oi import synth
+    data = open(src, "rb").read()
+    fields = {name: (off, size) for name, off, size in gguf_fields(data)}
+    where = gguf_tensor_data(data)
+    head = bytearray(data[:fields["end"][0]])
+    start = min(at for at, _ in where.values())
+    body = b""
+    for name, (at, kind) in sorted(where.items(), key=lambda t: t[1][0]):
+        nd = int.from_bytes(data[fields["tensor:%s.n_dims" % name][0]:][:4], "little")
+        dims = [int.from_bytes(data[fields["tensor:%s.dim%d" % (name, d)][0]:][:8], "little") for d in range(nd)]
+        rows = int(np.prod(dims[1:]))
+        size = rows * refcpu.row_byte_size(kind, dims[0])
+        raw = np.frombuffer(data, np.uint8, size, at)
+        new = next((k for end, k in kinds.items() if name.endswith(end)), kind)
+        if new != kind:
+            values = np.stack([refcpu.dequant_row(kind, r, dims[0]) for r in raw.reshape(rows, -1)])
+            raw = synth.quantize_rows(new, values)
+        off = fields["tensor:%s.offset" % name][0]
+        head[off - 4:off + 8] = struct.pack("<IQ", int(new), len(body))
+        body += raw.tobytes() + bytes(-raw.size % 32)
+    with open(dst, "wb") as f:
+        f.write(bytes(head) + bytes(start - len(head)) + body)

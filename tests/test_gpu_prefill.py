@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 import refcpu
-from helpers import scaled_err
+from helpers import gguf_retype, scaled_err
 from oi import _native, infer
 
 pytestmark = pytest.mark.gpu
@@ -198,6 +198,23 @@ def test_prefill_chunk_after_a_long_prompt(make_model, name, n):
         got = infer.engine_forward_batch(e, toks[600:], 600).copy()
         err = scaled_err(got, r.prefill(toks[600:], 600))
         assert err <= TOL, "scaled error %.3g" % err
+    finally:
+        infer.engine_destroy(e)
+        r.close()
+
+
+@pytest.mark.parametrize("n", [2, 7, 13])
+def test_trailing_tokens_of_gate_and_up_in_different_types(make_model, tmp_path, n):
+    """Gate in Q4_K and up in Q6_K: a prompt's and a draft's 2-7 trailing tokens
+    (13: a chunk of 8, then 5) are taken as the token step takes such a pair."""
+    path = str(tmp_path / "mixed.gguf")
+    gguf_retype(make_model("tiny-q4_k"), path, {"ffn_up.weight": 14})
+    e, r = _engines(path, 64)
+    try:
+        toks = _tokens(n, n, r.vocab_size)
+        rows = infer.engine_verify_batch(e, toks, 0).copy()
+        assert scaled_err(infer.engine_forward_batch(e, toks, 0), r.prefill(toks, 0)) <= TOL
+        assert scaled_err(rows, r.verify_batch(toks, 0)) <= TOL
     finally:
         infer.engine_destroy(e)
         r.close()
