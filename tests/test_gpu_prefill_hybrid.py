@@ -493,3 +493,22 @@ def test_few_tokens_equal_the_token_step(make_model, name, n):
     finally:
         infer.engine_destroy(e)
         infer.engine_destroy(s)
+
+
+@pytest.mark.parametrize("prompt", [0, 8])
+def test_two_trailing_tokens_of_a_routed_model_are_token_steps(make_model, prompt):
+    """Two trailing tokens of a routed model (alone, and after a chunk of 8) run
+    one at a time: their rows are the token step's, bit for bit."""
+    path = make_model("moe-tiny")
+    opts = infer.Engine_Opts(max_ctx=64)
+    (e, _), (s, _) = infer.engine_load(path, opts), infer.engine_load(path, opts)
+    try:
+        t = _tokens(9, prompt + 2, e.config.vocab_size)
+        rows = infer.engine_verify_batch(e, t, 0).copy()
+        if prompt:
+            infer.engine_forward_batch(s, t[:prompt], 0)
+        for i in range(prompt, prompt + 2):
+            assert np.array_equal(rows[i], infer.engine_forward(s, int(t[i]), i))
+    finally:
+        infer.engine_destroy(e)
+        infer.engine_destroy(s)
