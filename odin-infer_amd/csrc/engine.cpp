@@ -1573,8 +1573,8 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
 
 // The trailing 2-7 tokens of a call in one pass over the layers, in the arithmetic
 // of the token step (f32 activations, nothing staged in half): its GEMVs for all
-// the tokens at once (launch_gemv_nt), the chunk's attention, DeltaNet (token by
-// token) and routed experts between them.  Each trailing token through the token
+// the tokens at once (launch_gemv_nt), f32 attention, DeltaNet (token by token) and
+// routed experts between them.  Each trailing token through the token
 // step reads every weight again: five tokens of the 8B shape took 5 x 1.85 ms.
 int prefill_few(oi_engine *e, const int32_t *tokens, int T, int pos, float *rows) {
     const hipStream_t st = e->stream;
@@ -1628,8 +1628,8 @@ int prefill_few(oi_engine *e, const int32_t *tokens, int T, int pos, float *rows
                              (int32_t)c.n_kv_heads};
                 HIP_TRY(launch_pf_q35_qkv(qa, hd, st));
             }
-            HIP_TRY(launch_pf_attn(e->pf_q, L.kc, L.vc, nullptr, T, pos, (int)c.seq_len, (int)c.n_heads, (int)c.n_kv_heads,
-                                   hd, st, L.kind == LK_FULL ? e->pf_gate : nullptr, P[1], PB[1], act));
+            HIP_TRY(launch_pf_few_attn(e->pf_q, L.kc, L.vc, act, T, pos, (int)c.seq_len, (int)c.n_heads, (int)c.n_kv_heads,
+                                       hd, st, L.kind == LK_FULL ? e->pf_gate : nullptr, P[1], PB[1]));
             HIP_TRY(nt(GEMV_ADD, act, nullptr, {{&L.wo, e->pf_x}}));
         }
         if (L.moe) {

@@ -212,18 +212,13 @@ struct PfAttnArgs {
     uint16_t *out;              // [T][n_heads * head_dim] f16 (the wo projection's input)
     int32_t pos0, seq_len, n_heads, n_kv_heads;
     const float *gate;          // null, or [T][n_heads * head_dim]: out *= sigmoid(gate) (Qwen3.5)
-    float *out32;               // null, or f32 rows in place of out's
+    float *out32;               // null, or f32 rows in place of out's (pf_few_attn_kernel)
 };
 
 // the attention output of one element, gated when the layer has a gate
 static __device__ __forceinline__ float pf_gated(const PfAttnArgs &a, float o, size_t i) {
 #pragma clang fp contract(off)
     return a.gate ? o * sigmoid_ref(a.gate[i]) : o;
-}
-static __device__ __forceinline__ void pf_put(const PfAttnArgs &a, float o, size_t i) {
-    const float v = pf_gated(a, o, i);
-    if (a.out32) a.out32[i] = v;
-    else a.out[i] = f2h(v);
 }
 
 // Causal attention of token t (query head h, grid (n_heads, T)) over positions
@@ -304,7 +299,7 @@ __global__ __launch_bounds__(WG) void pf_attn_kernel(PfAttnArgs a) {
         float acc = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; w++) acc += ow[w][i] * sc[w];
-        pf_put(a, acc / lt, (size_t)t * QD + h * HD + i);
+        a.out[(size_t)t * QD + h * HD + i] = f2h(pf_gated(a, acc / lt, (size_t)t * QD + h * HD + i));
     }
 }
 
@@ -503,10 +498,6 @@ __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float
             float r[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) r[e] = pf_gated(a, o[dt][e] / lsum, d0 + 16 * dt + e);
-            if (a.out32) {
-                *(float4 *)(a.out32 + d0 + 16 * dt) = make_float4(r[0], r[1], r[2], r[3]);
-                continue;
-            }
             const uint32_t w0 = (uint32_t)f2h(r[0]) | ((uint32_t)f2h(r[1]) << 16);
             const uint32_t w1 = (uint32_t)f2h(r[2]) | ((uint32_t)f2h(r[3]) << 16);
             *(u32x2 *)(dst + 16 * dt) = u32x2{w0, w1};
@@ -514,7 +505,111 @@ __global__ __launch_bounds__(WG) void pf_fattn_kernel(PfAttnArgs a, int T, float
     }
 }
 
-// The splits of pf_fattn_kernel<HD, true>, a wave per (token, head) pair p = t
+// Attention of the few trailing tokens (T <= 16 queries) in the token step's f32
+// arithmetic: the tokens' queries are the columns of v_mfma_f32_16x16x4_f32, with
+// every score and weight an f32 (pf_fattn_kernel's halves keep 22 bits of a weight
+// and nothing below 2^-25, where the token step keeps 24 of any).  Wave z of the nz
+// waves of a head walks its range of 16-key tiles alone, with no LDS and no barrier,
+// the next tile's K and V rows on their way, and writes its (o, m, l) as split z for
+// pf_fattn_merge_kernel.  Lane (q, g) of S^T = K Q^T holds keys 4g + e of the tile
+// for query q, which is the B operand of O^T += V^T P^T when step e of that product
+// takes keys 4g + e; its A operand is element dt of the NDT consecutive dimensions
+// NDT q .. that the lane loaded of each of those rows, so row i of tile dt stands for
+// dimension NDT i + dt.  Bound by the products (HD / 2 of 32 clocks per tile and
+// wave) and, at short caches, by the two round trips before them.
+template <int HD>
+__global__ __launch_bounds__(WG) void pf_few_attn_kernel(PfAttnArgs a, int T, int nz, float *ws) {
+    constexpr int NC = HD / 32, NDT = HD / 16;
+    const int lane = threadIdx.x & (WAVE - 1), q = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x, z = (int)blockIdx.y * (WG / WAVE) + (int)threadIdx.x / WAVE;
+    if (z >= nz) return;
+    const int QD = a.n_heads * HD, kvh = h / (a.n_heads / a.n_kv_heads), tq = min(q, T - 1), qpos = a.pos0 + tq;
+    const int lmax = a.pos0 + T, nt = (lmax + 15) / 16, kt0 = (int)((long)nt * z / nz), kt1 = (int)((long)nt * (z + 1) / nz);
+    const uint16_t *kc = a.kc + (size_t)kvh * a.seq_len * HD, *vc = a.vc + (size_t)kvh * a.seq_len * HD;
+    struct Tile {
+        u32x4 k[NC], v[4][NDT / 8];
+    };
+    // (rows past the written range re-read the last written row; their scores are masked)
+    auto fetch = [&](int kt, Tile &r) {
+        const uint16_t *kr = kc + (size_t)min(16 * kt + q, lmax - 1) * HD + 8 * g;
+#pragma unroll
+        for (int c = 0; c < NC; c++) r.k[c] = *(const u32x4 *)(kr + 32 * c);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint16_t *vr = vc + (size_t)min(16 * kt + 4 * g + e, lmax - 1) * HD + NDT * q;
+#pragma unroll
+            for (int i = 0; i < NDT / 8; i++) r.v[e][i] = *(const u32x4 *)(vr + 8 * i);
+        }
+    };
+    auto half_of = [](const u32x4 &w, int e) { return h2f((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu); };
+    float4 qv[NC][2];
+    const float *qr = a.q + (size_t)tq * QD + h * HD + 8 * g;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        qv[c][0] = *(const float4 *)(qr + 32 * c);
+        qv[c][1] = *(const float4 *)(qr + 32 * c + 4);
+    }
+    const float rs = sqrtf((float)HD);
+    float m = -INFINITY, lsum = 0.f;
+    f32x4v o[NDT];
+#pragma unroll
+    for (int dt = 0; dt < NDT; dt++) o[dt] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    Tile cur, next;
+    fetch(kt0, cur);
+    for (int kt = kt0; kt < kt1; kt++) {
+        fetch(min(kt + 1, kt1 - 1), next);
+        f32x4v acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two chains
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float4 &v = qv[c][e >> 2];
+                const float qe = (e & 3) == 0 ? v.x : (e & 3) == 1 ? v.y : (e & 3) == 2 ? v.z : v.w;
+                acc[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(cur.k[c], e), qe, acc[e & 1], 0, 0, 0);
+            }
+        float s[4], bm = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            s[e] = 16 * kt + 4 * g + e <= qpos ? (acc[0][e] + acc[1][e]) / rs : -INFINITY;
+            bm = fmaxf(bm, s[e]);
+        }
+        bm = fmaxf(bm, __shfl_xor(bm, 16, WAVE));
+        bm = fmaxf(bm, __shfl_xor(bm, 32, WAVE));
+        // (no key of the range visible to this query yet: m and mn stay -inf)
+        const float mn = fmaxf(m, bm), alpha = mn == -INFINITY ? 1.f : expf(m - mn);
+        m = mn;
+        float ps = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            s[e] = mn == -INFINITY ? 0.f : expf(s[e] - mn);
+            ps += s[e];
+        }
+        lsum = lsum * alpha + ps;
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++) o[dt] *= alpha;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++)
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_of(cur.v[e][dt / 8], dt & 7), s[e], o[dt], 0, 0, 0);
+        cur = next;
+    }
+    lsum += __shfl_xor(lsum, 16, WAVE);
+    lsum += __shfl_xor(lsum, 32, WAVE);
+    if (q >= T) return;
+    float *pp = ws + (((size_t)z * T + q) * a.n_heads + h) * (HD + 2);
+#pragma unroll
+    for (int e = 0; e < 4; e++)  // row i = 4g + e of every tile: NDT consecutive dimensions
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt += 4)
+            *(float4 *)(pp + NDT * (4 * g + e) + dt) = make_float4(o[dt][e], o[dt + 1][e], o[dt + 2][e], o[dt + 3][e]);
+    if (g == 0) {
+        pp[HD] = m;
+        pp[HD + 1] = lsum;
+    }
+}
+
+// The splits of pf_fattn_kernel<HD, true> or pf_few_attn_kernel, a wave per (token, head) pair p = t
 // n_heads + h: O = sum_s e^{m_s - M} o_s / sum_s e^{m_s - M} l_s.  Lane z holds split
 // z's m and l (at most 64 splits); the weighted sums of the lane's HD / 64 dimensions run over
 // four splits' loads at a time.
@@ -552,7 +647,9 @@ __global__ __launch_bounds__(WG) void pf_fattn_merge_kernel(PfAttnArgs a, int T,
 #pragma unroll
     for (int e = 0; e < DPL; e++) {
         const size_t i = (size_t)p * HD + lane + WAVE * e;
-        pf_put(a, O[e] / L, i);
+        const float v = pf_gated(a, O[e] / L, i);
+        if (a.out32) a.out32[i] = v;
+        else a.out[i] = f2h(v);
     }
 }
 
@@ -594,8 +691,8 @@ hipError_t launch_pf_qkv(const PfQkvArgs &a, int head_dim, hipStream_t st) {
 
 hipError_t launch_pf_attn(const float *q, const uint16_t *kc, const uint16_t *vc, uint16_t *out, int T, int pos0,
                           int seq_len, int n_heads, int n_kv_heads, int head_dim, hipStream_t st, const float *gate,
-                          float *ws, size_t ws_bytes, float *out32) {
-    PfAttnArgs a{q, kc, vc, out, pos0, seq_len, n_heads, n_kv_heads, gate, out32};
+                          float *ws, size_t ws_bytes) {
+    PfAttnArgs a{q, kc, vc, out, pos0, seq_len, n_heads, n_kv_heads, gate, nullptr};
     const dim3 grid((unsigned)n_heads, (unsigned)T);
     const dim3 fgrid((unsigned)n_heads, (unsigned)((T + 63) / 64));
     // The key blocks of a query tile are split over workgroups where the tiles
@@ -626,6 +723,28 @@ hipError_t launch_pf_attn(const float *q, const uint16_t *kc, const uint16_t *vc
         hipLaunchKernelGGL((pf_fattn_kernel<256>), fgrid, dim3(WG), 0, st, a, T, nullptr);
     else if (head_dim == 256) hipLaunchKernelGGL(pf_attn_kernel<256>, grid, dim3(WG), 0, st, a);
     else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// Two waves per SIMD where each still has two tiles of keys, and as many splits as
+// the scratch holds (the merge takes 64).
+hipError_t launch_pf_few_attn(const float *q, const uint16_t *kc, const uint16_t *vc, float *out, int T, int pos0, int seq_len,
+                              int n_heads, int n_kv_heads, int head_dim, hipStream_t st, const float *gate, float *ws,
+                              size_t ws_bytes) {
+    const size_t per = (size_t)T * n_heads * (head_dim + 2) * 4;
+    if (T < 1 || T > 16 || !ws || ws_bytes < per) return hipErrorInvalidValue;
+    const PfAttnArgs a{q, kc, vc, nullptr, pos0, seq_len, n_heads, n_kv_heads, gate, out};
+    const int nt = (pos0 + T + 15) / 16;
+    const int nz = std::max(1, std::min({64, nt / 2, (2048 + n_heads - 1) / n_heads, (int)std::min<size_t>(ws_bytes / per, 64)}));
+    const dim3 grid((unsigned)n_heads, (unsigned)((nz + WG / WAVE - 1) / (WG / WAVE)));
+    const dim3 mgrid((unsigned)((T * n_heads + WG / WAVE - 1) / (WG / WAVE)));
+    if (head_dim == 128) {
+        hipLaunchKernelGGL(pf_few_attn_kernel<128>, grid, dim3(WG), 0, st, a, T, nz, ws);
+        hipLaunchKernelGGL(pf_fattn_merge_kernel<128>, mgrid, dim3(WG), 0, st, a, T, (const float *)ws, nz);
+    } else if (head_dim == 256) {
+        hipLaunchKernelGGL(pf_few_attn_kernel<256>, grid, dim3(WG), 0, st, a, T, nz, ws);
+        hipLaunchKernelGGL(pf_fattn_merge_kernel<256>, mgrid, dim3(WG), 0, st, a, T, (const float *)ws, nz);
+    } else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -20,7 +20,7 @@ import pytest
 
 import refcpu
 from helpers import gguf_tensor_data, scaled_err
-from oi import infer
+from oi import infer, synth
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -470,26 +470,93 @@ def test_verify_batch_vs_oracle(make_model, name, seed):
 
 
 @pytest.mark.parametrize("name", ["tiny-q4_k", "tiny-q8_0", "moe-tiny", "qwen35-tiny", "qwen35-moe-tiny", "8b-1layer-q4_k"])
-@pytest.mark.parametrize("n", [2, 3, 5, 7])
-def test_few_tokens_equal_the_token_step(make_model, name, n):
+@pytest.mark.parametrize("n,pos", [(2, 24), (3, 24), (5, 24), (7, 24), (3, 616), (7, 616)])
+def test_few_tokens_equal_the_token_step(make_model, name, n, pos):
     """2-7 tokens in one pass (every row's logits) against the same tokens through
     the token step on a second engine: the same arithmetic in another order (the
-    8B shape's 12288-column rows run in three passes), so the rows differ by f32
+    8B shape's 12288-column rows run in three passes; after 616 positions the
+    attention merges 19 ranges of keys, at 24 it has one), so the rows differ by f32
     rounding and by the f16 cache values that it tips over: 2^-11 of a few cached
     values of a few hundred, below 5e-4 of the largest logit.  The states after
-    are the same to that measure, and a row is the same in a shorter call."""
+    are the same to that measure."""
     path = make_model(name)
-    opts = infer.Engine_Opts(max_ctx=128)
+    opts = infer.Engine_Opts(max_ctx=pos + 16)
     (e, _), (s, _) = infer.engine_load(path, opts), infer.engine_load(path, opts)
     try:
-        t = _tokens(n + 1, 24 + n, e.config.vocab_size)
+        t = _tokens(n + 1, pos + n, e.config.vocab_size)
         for x in (e, s):
-            infer.engine_forward_batch(x, t[:24], 0)
-        rows = infer.engine_verify_batch(e, t[24:], 24).copy()
-        ref = np.array([infer.engine_forward(s, int(t[24 + i]), 24 + i).copy() for i in range(n)])
+            infer.engine_forward_batch(x, t[:pos], 0)
+        rows = infer.engine_verify_batch(e, t[pos:], pos).copy()
+        ref = np.array([infer.engine_forward(s, int(t[pos + i]), pos + i).copy() for i in range(n)])
         errs = [scaled_err(rows[i], ref[i]) for i in range(n)]
         assert max(errs) <= 5e-4, errs
-        assert scaled_err(infer.engine_forward(e, 5, 24 + n), infer.engine_forward(s, 5, 24 + n)) <= 5e-4
+        assert scaled_err(infer.engine_forward(e, 5, pos + n), infer.engine_forward(s, 5, pos + n)) <= 5e-4
+    finally:
+        infer.engine_destroy(e)
+        infer.engine_destroy(s)
+
+
+def _first_queries(path, spec, tokens, pos):
+    """The first layer's rotated queries of `tokens` at `pos`, `pos` + 1, .. as
+    [token][head][head_dim], in float64 from the file."""
+    data = open(path, "rb").read()
+    where = gguf_tensor_data(data)
+
+    def rows(name, n, picked):
+        at, kind = where[name]
+        size = refcpu.row_byte_size(kind, n)
+        return np.stack([refcpu.dequant_row(kind, np.frombuffer(data, np.uint8, size, at + size * int(i)), n)
+                         for i in picked]).astype(np.float64)
+
+    d, h, hd = spec["dim"], spec["n_heads"], spec["head_dim"]
+
+    def norm(x, name):
+        w = rows(name, x.shape[-1], [0])[0]
+        return w * x / np.sqrt((x * x).mean(-1, keepdims=True) + spec["rms_eps"])
+
+    x = norm(rows("token_embd.weight", d, tokens), "blk.0.attn_norm.weight")
+    q = norm((x @ rows("blk.0.attn_q.weight", d, range(h * hd)).T).reshape(-1, h, hd), "blk.0.attn_q_norm.weight")
+    half = hd // 2
+    a = (pos + np.arange(len(tokens)))[:, None, None] * spec["rope_theta"] ** (-np.arange(half) / half)
+    u, v = q[..., :half], q[..., half:]
+    return np.concatenate([u * np.cos(a) - v * np.sin(a), u * np.sin(a) + v * np.cos(a)], -1)
+
+
+@pytest.mark.parametrize("hd,kv", [(128, 2), (256, 1)])
+@pytest.mark.parametrize("gap,pos", [(21, 610), (12, 610), (18, 70)])
+def test_few_tokens_keep_small_weights(make_model, hd, kv, gap, pos):
+    """Keys that draw `gap` more than all others and whose values are zero, as an
+    attention sink's: the output is made of weights of e^-gap (2^-30 at 21) alone, times
+    values of 20000.  The token step holds a weight in f32 whatever its size; two halves
+    lose one below 2^-25.  Measured as the effect on the logits against the
+    token step's: the same f32 arithmetic in another order, so sums of 600 terms
+    within 600 2^-24 = 4e-5 of their size, doubled through the layer."""
+    over = dict(n_layers=1, n_heads=4, n_kv_heads=kv, head_dim=hd)
+    path, n = make_model("tiny-q4_k", **over), 5
+    spec = dict(synth.CONFIGS["tiny-q4_k"], **over)
+    t = _tokens(gap, n, spec["vocab_size"])
+    q = _first_queries(path, spec, t, pos)
+    k16, v16 = np.zeros((1, kv, pos, hd), np.float16), np.full((1, kv, pos, hd), 20000, np.float16)
+    v16[:] *= np.where(np.arange(hd) % 3 == 0, -1, 1).astype(np.float16)
+    for g in range(kv):  # a key along each query of the group: score `gap` (q.q = hd up to the norm weights)
+        own = q[:, g * (4 // kv):(g + 1) * (4 // kv)].reshape(-1, hd)
+        at = 3 + 3 * np.arange(len(own))
+        k16[0, g, at] = own * (gap * np.sqrt(hd) / (own * own).sum(-1, keepdims=True))
+        v16[0, g, at] = 0
+    opts = infer.Engine_Opts(max_ctx=pos + 16)
+    (e, _), (s, _) = infer.engine_load(path, opts), infer.engine_load(path, opts)
+    try:
+        for x in (e, s):
+            infer.engine_kv_fill(x, 0, 0, k16.view(np.uint16), v16.view(np.uint16))
+        rows = infer.engine_verify_batch(e, t, pos).copy()
+        ref = np.array([infer.engine_forward(s, int(t[i]), pos + i).copy() for i in range(n)])
+        infer.engine_kv_fill(s, 0, 0, k16.view(np.uint16), np.zeros_like(v16).view(np.uint16))
+        without = np.array([infer.engine_forward(s, int(t[i]), pos + i).copy() for i in range(n)])
+        effect = [scaled_err(without[i], ref[i]) for i in range(n)]
+        errs = [scaled_err(rows[i], ref[i]) for i in range(n)]
+        print("hd %d gap %d: effect %.2g - %.2g, error %.2g" % (hd, gap, min(effect), max(effect), max(errs)))
+        assert min(effect) > 1e-2
+        assert max(errs) <= 8e-5, errs
     finally:
         infer.engine_destroy(e)
         infer.engine_destroy(s)
