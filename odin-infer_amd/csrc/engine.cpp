@@ -1560,12 +1560,14 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
             HIP_TRY(launch_pf_add(e->pf_x, P[0], s0, (int64_t)T * D, st));
     }
     // the final norm and classifier (qwen3_5/metal.odin:1637-1641 for the last token;
-    // metal_verify_batch_logits, qwen3_5/metal.odin:1707-1747, for every token)
-    if (rows) return prefill_classify(e, 0, T, rows);
+    // metal_verify_batch_logits, qwen3_5/metal.odin:1707-1747, for every token); the
+    // last token's logits are the same bits either way
+    if (rows && gemv_nt_repeats(e->output)) return prefill_classify(e, 0, T, rows);
+    if (rows && prefill_classify(e, 0, T - 1, rows)) return -1;
     GemvArgs a = gemv_args(GEMV_STORE, D, e->pf_x + (size_t)(T - 1) * D, e->output_norm, eps);
     a.nseg = 1;
     a.seg[0].m = e->output;
-    a.seg[0].y = e->logits;
+    a.seg[0].y = rows ? rows + (size_t)(T - 1) * c.vocab_size : e->logits;
     if (!plan_gemv(a)) return fail(OI_E_DEVICE, "internal: classifier plan");
     HIP_TRY(launch_gemv(a, st));
     return OI_OK;

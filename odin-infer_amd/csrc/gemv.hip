@@ -1166,7 +1166,7 @@ __global__ __launch_bounds__(NT_THREADS) void gemv_nt_kernel(GemvNtArgs a) {
     using W = typename Types<T>::W;
     using X = typename Types<T>::X;
     extern __shared__ u32x4 smem[];
-    __shared__ float red[GEMV_NT_MAX][NT_NW];
+    __shared__ float red[GEMV_NT_MAX][GNW];
     __shared__ float rsc[GEMV_NT_MAX];
     __shared__ uint32_t tile_ctr;
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
@@ -1222,14 +1222,20 @@ __global__ __launch_bounds__(NT_THREADS) void gemv_nt_kernel(GemvNtArgs a) {
             int to = t;
             asm volatile("" : "+s"(to));  // (the addresses of eight tokens' planes are not kept across passes)
             const XQ q = planes(to);
-            float ss = 0.f;
 #pragma unroll
             for (int i = 0; i < XP; i++) {
                 const int c = tid + i * NT_THREADS;  // (kl / 4 is a multiple of 64: whole waves)
-                if (c >= kl / 4) break;
+                if (c >= kl / 4) {
+                    if (NORM && k0 == 0 && lane == 0) red[t][wave + i * NT_NW] = 0.f;
+                    continue;
+                }
                 float4 v = xv[t][i];
                 if (NORM) {
+                    // the token step's sums: its wave w of 16 has the float4s 64 w ..
+                    float ss = 0.f;
                     ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+                    ss = wave_sum(ss);
+                    if (lane == 0) red[t][wave + i * NT_NW] = k0 > 0 ? red[t][wave + i * NT_NW] + ss : ss;
                     {
 #pragma clang fp contract(off)
                         v.x = nw[i].x * v.x;
@@ -1240,10 +1246,6 @@ __global__ __launch_bounds__(NT_THREADS) void gemv_nt_kernel(GemvNtArgs a) {
                 }
                 quant4(v, c, (uint32_t *)q.hi, (uint32_t *)q.mid, (uint32_t *)q.lo, (float *)q.xs, (float *)q.s32,
                        (float *)q.s16);
-            }
-            if (NORM) {
-                ss = wave_sum(ss);
-                if (lane == 0) red[t][wave] = k0 > 0 ? red[t][wave] + ss : ss;
             }
             __builtin_amdgcn_sched_barrier(0);  // (one token's quantization in registers at a time)
         }
@@ -1293,10 +1295,14 @@ __global__ __launch_bounds__(NT_THREADS) void gemv_nt_kernel(GemvNtArgs a) {
         }
     }
     if (NORM && tid < n) {
-        float s = 0.f;
+        float s[GNW / 2];  // in xpre_finish's order
 #pragma unroll
-        for (int i = 0; i < NT_NW; i++) s += red[tid][i];
-        rsc[tid] = 1.0f / sqrtf(s / (float)K + a.eps);
+        for (int i = 0; i < GNW / 2; i++) s[i] = red[tid][2 * i] + red[tid][2 * i + 1];
+#pragma unroll
+        for (int w = GNW / 4; w >= 1; w >>= 1)
+#pragma unroll
+            for (int i = 0; i < w; i++) s[i] = s[2 * i] + s[2 * i + 1];
+        rsc[tid] = 1.0f / sqrtf(s[0] / (float)K + a.eps);
     }
     __syncthreads();
     float *y = a.seg[seg].y;
@@ -1317,6 +1323,13 @@ __global__ __launch_bounds__(NT_THREADS) void gemv_nt_kernel(GemvNtArgs a) {
 
 bool gemv_nt_supported(const DMat &m) {
     return (m.type == T_Q4_K || m.type == T_Q6_K || m.type == T_Q8_0) && m.cols % 256 == 0;
+}
+
+// whether each row's result is the token step's, bit for bit: one pass, and a unit per
+// lane of a row, as launch_gemv_q has it for a power of two of units
+bool gemv_nt_repeats(const DMat &m) {
+    const int U = m.cols / 64;
+    return gemv_nt_supported(m) && U <= NT_KS / 64 && (U & (U - 1)) == 0;
 }
 
 template <int T, int R, int NM>

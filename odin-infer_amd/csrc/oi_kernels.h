@@ -222,6 +222,7 @@ struct GemvNtArgs {
 };
 // whether the kernel takes the matrices (one type and row length)
 bool gemv_nt_supported(const DMat &m);
+bool gemv_nt_repeats(const DMat &m);
 hipError_t launch_gemv_nt(GemvNtArgs a, hipStream_t st);
 
 // gemm.hip: batched projection c[t][r] = sum_k f16(deq(W))[r][k] x[t][k]

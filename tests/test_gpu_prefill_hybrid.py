@@ -579,3 +579,22 @@ def test_two_trailing_tokens_of_a_routed_model_are_token_steps(make_model, promp
     finally:
         infer.engine_destroy(e)
         infer.engine_destroy(s)
+
+
+@pytest.mark.parametrize("name,over", [("tiny-q8_0", {}), ("tiny-q4_k", {}), ("8b-1layer-q4_k", {}),
+                                       ("tiny-q4_k", dict(dim=768)), ("tiny-q4_k", dict(dim=5120, n_layers=1)),
+                                       ("qwen35-moe-tiny", {})])
+@pytest.mark.parametrize("n", [8, 24])
+def test_last_verified_row_is_the_prefills(make_model, name, over, n):
+    """A draft of whole chunks: its last row is the prompt call's result for the same
+    tokens, bit for bit, whether the classifier of every row sums in the token
+    step's order (rows of 256, 512 and 4096) or not (768, 5120)."""
+    path = make_model(name, **over)
+    opts = infer.Engine_Opts(max_ctx=64)
+    (e, _), (s, _) = infer.engine_load(path, opts), infer.engine_load(path, opts)
+    try:
+        t = _tokens(n, n, e.config.vocab_size)
+        assert np.array_equal(infer.engine_verify_batch(e, t, 0)[-1], infer.engine_forward_batch(s, t, 0))
+    finally:
+        infer.engine_destroy(e)
+        infer.engine_destroy(s)
