@@ -48,6 +48,8 @@
 //   D[i][j] (16 floats): j = l % 32, i = 8 (v / 4) + 4 (l / 32) + v % 4.
 
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
 
 #include "device_common.h"
 
@@ -504,18 +506,241 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q_kernel(GemmArgs a) {
     }
 }
 
-// c[i] = sum over slices z (in order) of part[z][i]; eight slices' loads are in
+// ---- 16-row waves ---------------------------------------------------------------
+// gemm_r_kernel: 128 rows x 64 tokens, wave w rows 16w .. 16w+15 of every chunk in
+// four v_mfma_f32_16x16x32_f16 accumulators (A[i][k]: i = l % 16, k = 8 (l / 16) + e;
+// D[i][j]: j = l % 16, i = 4 (l / 16) + e).  The weights go from memory straight into
+// the operand layout, one chunk ahead in registers: lane quarter q holds unit 4c + q
+// of its row, and the chunk's eight 32-wide K steps take 8 of its weights each.  Only
+// the activations are staged, so the first product waits for less, nothing is summed
+// at the end, and two workgroups fit a CU; against that every chunk takes longer
+// (the loads' address work, twice the matrix instructions).  The codes are converted
+// by v_cvt_f32_ubyte{0..3} here: codes8 measured 3 - 5% slower (4069 x 2816 Q6_K, 79
+// tokens: 14.3 us against 13.8).
+// keeps a masked word opaque, so that its bytes convert with v_cvt_f32_ubyte{0..3}
+// instead of being re-extracted one by one from the unmasked word
+static __device__ __forceinline__ uint32_t opaque(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+struct RQ4K {  // step st = 4h + 2p + b: nibble h, plane p, bytes 8b .. 8b+7; octet 8q + st
+    struct Src {
+        rsrc_t q, s;
+        uint32_t plane, qo, so;
+    };
+    struct Raw {
+        u32x4 p[2], hdr;
+    };
+    struct Pre {
+        float d1[2], mm[2];
+    };
+    static __device__ __forceinline__ Src src(const DMat &m, int row, int q) {
+        return Src{make_rsrc(m.q, 2 * m.plane), make_rsrc(m.s, (size_t)m.rows * (m.cols >> 8) * 16), (uint32_t)m.plane,
+                   (uint32_t)((row * (m.cols >> 6) + q) * 16), (uint32_t)(row * (m.cols >> 8) * 16)};
+    }
+    static __device__ __forceinline__ void raw(const Src &g, int c, Raw &r) {
+        r.p[0] = bld16(g.q, g.qo, 64 * c);
+        r.p[1] = bld16(g.q, g.qo + g.plane, 64 * c);
+        r.hdr = bld16(g.s, g.so, 16 * c);
+    }
+    static __device__ __forceinline__ Pre pre(const Raw &r, int q) {
+        const float d = h2f(r.hdr.x & 0xFFFFu), dmin = h2f(r.hdr.x >> 16);
+        uint32_t sc0, m0, sc1, m1;
+        q4k_scales(q, r.hdr.y, r.hdr.z, r.hdr.w, sc0, m0, sc1, m1);
+        return Pre{{d * (float)sc0, d * (float)sc1}, {dmin * (float)m0, dmin * (float)m1}};
+    }
+    static __device__ __forceinline__ h8 deq(const Raw &r, const Pre &p, int st) {
+        const int h = st >> 2, b = st & 1;
+        const u32x4 &w = r.p[(st >> 1) & 1];
+        const uint32_t lo = opaque(((b ? w.z : w.x) >> (4 * h)) & 0x0F0F0F0Fu);
+        const uint32_t hi = opaque(((b ? w.w : w.y) >> (4 * h)) & 0x0F0F0F0Fu);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = __builtin_fmaf(p.d1[h], (float)byte_of(lo, hi, e), -p.mm[h]);
+        return cvt8(v);
+    }
+};
+struct RQ6K {  // step st = 2s + b: run s, bytes 8b .. 8b+7; octet 16 (q / 2) + 4s + 2 (q % 2) + b
+    struct Src {
+        rsrc_t q, s, d;
+        uint32_t plane, qo, so, dof;
+    };
+    struct Raw {
+        u32x4 l[2], h;
+        u32x2 sc;
+        uint32_t d;
+    };
+    struct Pre {
+        float ds[4], off[4];
+    };
+    static __device__ __forceinline__ Src src(const DMat &m, int row, int q) {
+        const int nsb = m.cols >> 8;
+        return Src{make_rsrc(m.q, 3 * m.plane), make_rsrc(m.s, (size_t)m.rows * nsb * 16),
+                   make_rsrc(m.d, (size_t)m.rows * nsb * 2), (uint32_t)m.plane, (uint32_t)((row * (m.cols >> 6) + q) * 16),
+                   (uint32_t)(row * nsb * 16 + 8 * (q >> 1)), (uint32_t)(row * nsb * 2)};
+    }
+    static __device__ __forceinline__ void raw(const Src &g, int c, Raw &r) {
+        r.l[0] = bld16(g.q, g.qo, 64 * c);
+        r.l[1] = bld16(g.q, g.qo + g.plane, 64 * c);
+        r.h = bld16(g.q, g.qo + 2 * g.plane, 64 * c);
+        r.sc = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(g.s, g.so, 16 * c, 0));
+        r.d = __builtin_amdgcn_raw_buffer_load_b16(g.d, g.dof, 2 * c, 0);
+    }
+    static __device__ __forceinline__ Pre pre(const Raw &r, int q) {
+        Pre p;
+        const float d = h2f(r.d);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            p.ds[s] = d * (float)(int8_t)byte_of(r.sc.x, r.sc.y, (q & 1) + 2 * s);
+            p.off[s] = -32.f * p.ds[s];
+        }
+        return p;
+    }
+    static __device__ __forceinline__ h8 deq(const Raw &r, const Pre &p, int st) {
+        const int s = st >> 1, b = st & 1;
+        const u32x4 &l = r.l[s & 1];
+        const uint32_t llo = ((b ? l.z : l.x) >> (4 * (s >> 1))) & 0x0F0F0F0Fu;
+        const uint32_t lhi = ((b ? l.w : l.y) >> (4 * (s >> 1))) & 0x0F0F0F0Fu;
+        const uint32_t hlo = (((b ? r.h.z : r.h.x) >> (2 * s)) & 0x03030303u) << 4;
+        const uint32_t hhi = (((b ? r.h.w : r.h.y) >> (2 * s)) & 0x03030303u) << 4;
+        const uint32_t wlo = opaque(llo | hlo), whi = opaque(lhi | hhi);  // 6-bit codes, one per byte
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = __builtin_fmaf(p.ds[s], (float)byte_of(wlo, whi, e), p.off[s]);
+        return cvt8(v);
+    }
+};
+struct RQ80 {  // step st = 4 blk + 2 half + b: octet 8q + st
+    struct Src {
+        rsrc_t q, d;
+        uint32_t plane, qo, dof;
+    };
+    struct Raw {
+        u32x4 p[4];
+        uint32_t d;
+    };
+    struct Pre {
+        float d[2];
+    };
+    static __device__ __forceinline__ Src src(const DMat &m, int row, int q) {
+        return Src{make_rsrc(m.q, 4 * m.plane), make_rsrc(m.d, (size_t)m.rows * (m.cols >> 5) * 2), (uint32_t)m.plane,
+                   (uint32_t)((row * (m.cols >> 6) + q) * 16), (uint32_t)((row * (m.cols >> 5) + 2 * q) * 2)};
+    }
+    static __device__ __forceinline__ void raw(const Src &g, int c, Raw &r) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) r.p[k] = bld16(g.q, g.qo + k * g.plane, 64 * c);
+        r.d = __builtin_amdgcn_raw_buffer_load_b32(g.d, g.dof, 16 * c, 0);
+    }
+    static __device__ __forceinline__ Pre pre(const Raw &r, int) { return Pre{{h2f(r.d & 0xFFFFu), h2f(r.d >> 16)}}; }
+    static __device__ __forceinline__ h8 deq(const Raw &r, const Pre &p, int st) {
+#pragma clang fp contract(off)
+        const u32x4 &w = r.p[st >> 1];
+        const uint32_t lo = (st & 1) ? w.z : w.x, hi = (st & 1) ? w.w : w.y;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = p.d[st >> 2] * (float)(int8_t)byte_of(lo, hi, e);
+        return cvt8(v);
+    }
+};
+
+template <class G, class R>
+__global__ __launch_bounds__(GM_THREADS) void gemm_r_kernel(GemmArgs a) {
+    constexpr int TOK = 64, XV = TOK * GM_KC / 8, XPT = XV / GM_THREADS;
+    __shared__ __attribute__((aligned(16))) u32x4 xs[2][XV];  // as gemm_q_kernel's
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE, q = lane >> 4, li = lane & 15;
+    // one projection: grid (row tiles, token tiles, K slices), else flat
+    int sg = 0, bx = (int)blockIdx.x, by = (int)blockIdx.y, bz = (int)blockIdx.z;
+    if (a.nseg > 1) {
+#pragma unroll
+        for (int i = 1; i < GM_MAX_SEG; i++)
+            if (i < a.nseg && bx >= a.seg[i].first) sg = i;
+        const int nx = a.seg[sg].nx, ny = (a.n + TOK - 1) / TOK, loc = bx - a.seg[sg].first;
+        bz = loc / (nx * ny);
+        by = (loc - bz * nx * ny) / nx;
+        bx = loc - (bz * ny + by) * nx;
+    }
+    const GemmSeg &g = a.seg[sg];
+    const DMat &mat = g.m;
+    const int t0 = by * TOK;
+    const int M = mat.rows, K = mat.cols, c0 = bz * g.cps, c1 = min(K / GM_KC, c0 + g.cps);
+    const typename R::Src src = R::src(mat, min(bx * GM_ROWS + 16 * wave + li, M - 1), q);  // rows past M: not stored
+
+    const rsrc_t xsrc = make_rsrc(a.x, (size_t)a.n * K * 2);
+    uint32_t xoff[XPT];
+#pragma unroll
+    for (int i = 0; i < XPT; i++) {
+        const int p = tid + i * GM_THREADS;
+        xoff[i] = (uint32_t)(min(t0 + (p >> 5), a.n - 1) * K * 2 + 16 * (p & 31));
+    }
+    u32x4 xr[XPT];
+    auto xfetch = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < XPT; i++) xr[i] = bld16(xsrc, xoff[i], c * GM_KC * 2);
+    };
+    f32x4v acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    typename R::Raw ring[2];
+    if (c0 < c1) {
+        R::raw(src, c0, ring[0]);
+        xfetch(c0);
+    }
+    for (int cb = c0; cb < c1; cb += 2) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int c = cb + r;
+            if (c >= c1) break;
+            R::raw(src, c + 1 < c1 ? c + 1 : c0, ring[r ^ 1]);  // (past the slice: its first chunk, unused)
+#pragma unroll
+            for (int i = 0; i < XPT; i++) {
+                const int p = tid + i * GM_THREADS, j = p >> 5, o = p & 31;
+                xs[r][o * TOK + (j ^ (o & 7))] = xr[i];
+            }
+            if (c + 1 < c1) xfetch(c + 1);
+            __syncthreads();  // chunk c staged; every wave is done with chunk c - 2's buffer
+            const typename R::Pre pre = R::pre(ring[r], q);
+#pragma unroll
+            for (int st = 0; st < 8; st++) {
+                const int o = G::octet(q, st);
+                h8 B[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) B[t] = __builtin_bit_cast(h8, xs[r][o * TOK + ((16 * t + li) ^ (o & 7))]);
+                const h8 A = R::deq(ring[r], pre, st);
+#pragma unroll
+                for (int t = 0; t < 4; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[t], acc[t], 0, 0, 0);
+            }
+        }
+    }
+    // lane (j, q) of tile t holds rows 4q .. 4q+3 of token 16t + j
+    const int r0 = bx * GM_ROWS + 16 * wave + 4 * q;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int tk = t0 + 16 * t + li;
+        if (tk >= a.n) continue;
+        float *dst = g.c + ((size_t)bz * a.n + tk) * M + r0;
+        if (r0 + 3 < M && (M & 3) == 0) {
+            *(f32x4v *)dst = acc[t];
+            continue;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (r0 + e < M) dst[e] = acc[t][e];
+    }
+}
+
+// c[i] = sum over slices z (in order) of part[z][i]; NB slices' loads are in
 // flight together (a loop of load and add waits for each in turn)
+template <int NB>
 __global__ __launch_bounds__(WG) void gemm_reduce(const float *part, float *c, int64_t total, int split) {
     const int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x;
     if (4 * i + 3 < total) {
         f32x4v s = {0.f, 0.f, 0.f, 0.f};
-        for (int z0 = 0; z0 < split; z0 += 8) {
-            f32x4v v[8];
+        for (int z0 = 0; z0 < split; z0 += NB) {
+            f32x4v v[NB];
 #pragma unroll
-            for (int k = 0; k < 8; k++) v[k] = *(const f32x4v *)(part + min(z0 + k, split - 1) * total + 4 * i);
+            for (int k = 0; k < NB; k++) v[k] = *(const f32x4v *)(part + min(z0 + k, split - 1) * total + 4 * i);
 #pragma unroll
-            for (int k = 0; k < 8; k++)
+            for (int k = 0; k < NB; k++)
                 if (z0 + k < split) s = z0 + k ? s + v[k] : v[k];
         }
         *(f32x4v *)(c + 4 * i) = s;
@@ -532,43 +757,60 @@ bool gemm_supported(const DMat &m) {
     return (m.type == T_Q4_K || m.type == T_Q6_K || m.type == T_Q8_0) && m.cols % GM_KC == 0;
 }
 
-static int normalize_split(int nchunk, int split) {
-    const int cps = (nchunk + split - 1) / split;
-    return (nchunk + cps - 1) / cps;
-}
-
-// Token tiles (of 16) per workgroup and K split of a launch of `rt` row tiles: the
-// pair of least estimated time with at most `cap` slices.  The estimate (us) has a
+// Kernel, token tiles (of 16) per workgroup and K split of a launch of `rt` row tiles:
+// those of least estimated time with at most `cap` slices.  The estimate (us) has a
 // CU's workgroups one after another (two of 32 tokens fit a CU, and take twice as
-// long): a chunk and a fixed time per workgroup, every slice written and read back,
-// and the reduction's launch if the caller has one.  Its constants are fitted to
-// 240 shapes (500 - 12288 rows, 1024 - 12288 columns, 8 - 512 tokens, the three
-// types) run at every tile and 11 splits: the chosen pair takes 1.4% (Q4_K), 0.4%
-// (Q6_K) and 0.2% (Q8_0) longer than the fastest one on average.  With the tile
-// taken from n alone (32 tokens up to 32, 64 or 128 above) and the constants of
-// two large matrices it was 4.1, 3.0 and 2.6%, and up to 41%: few rows or columns
+// long; a second one of gemm_r_kernel's adds 0.8 of the first): a chunk and a fixed
+// time per workgroup, every slice written and read back, and the reduction's launch
+// if the caller has one.  Its constants are fitted to 210 shapes (500 - 12288 rows,
+// 1024 - 12288 columns, 8 - 512 tokens, the three types) run with every kernel and
+// tile at two or three splits, on three sets of inputs in turn: the choice takes 1.8%
+// (Q4_K), 1.4% (Q6_K) and 1.7% (Q8_0) longer than the fastest one on average.
+// gemm_r_kernel wins where up to 64 tokens fill 150 workgroups or more (the weights'
+// stream bounds it: 4096 x 4096 Q4_K, 64 tokens: 11.8 us against 12.5), and where whole
+// tiles of 64 tokens fill every CU once with few chunks, or once and a half with many.
+// Without it 37 of the shapes took over 2% longer than with it alone (up to 15%, for
+// 8% less on average); now 5 do, up to 6% in all but one.  With the tile taken from n
+// alone (32 tokens up to 32, 64 or 128 above) it was up to 41%: few rows or columns
 // want more and smaller tiles at any n (3095 x 1024 Q4_K, 157 tokens: 9.1 us at 32
-// tokens a tile, 10.6 at 64).  Tiles of 96 tokens are worth 3.5% on average for
-// Q8_0, which has no larger one, and 0.7% for the others.
+// tokens a tile, 10.6 at 64).  Tiles of 96 tokens are worth 3.5% on average for Q8_0,
+// which has no larger one, and 0.7% for the others.
 struct GemmPlan {
     int tt, split;
+    bool r16;  // gemm_r_kernel (tt 4)
 };
-static GemmPlan gemm_plan(int type, int rt, int nchunk, int32_t n, double out, int cap, bool reduce) {
-    GemmPlan best{2, 1};
-    double bt = 1e30;
+static GemmPlan gemm_plan(int type, int rt, int nchunk, int32_t n, double out, int cap, bool reduce, bool pair = false) {
+    const char *only = std::getenv("OI_GEMM_TILE");  // 32, 64, 96, 128 tokens or "r16": that kernel alone (tests)
     const double unit = type == T_Q4_K ? 0.9 : 1.0;  // (the fewest instructions per weight)
-    for (int tt : {2, 4, 6, 8}) {
-        if (tt == 8 && type == T_Q8_0) continue;
-        const double chunk = unit * (tt == 8 ? 1.9 : tt == 6 ? 1.78 : tt == 4 ? 1.65 : 1.35);
-        const double fixed = tt == 8 ? 6.3 : tt == 6 ? 4.5 : tt == 4 ? 2.9 : 2.2;
-        const int tiles = rt * ((n + 16 * tt - 1) / (16 * tt));
-        for (int s = 1; s <= std::max(1, nchunk / 2) && s <= cap; s++) {
-            if (normalize_split(nchunk, s) != s) continue;
-            const double t = (tiles * s + 255) / 256 * (((nchunk + s - 1) / s) * chunk + fixed) +
-                             (s > 1 ? s * out * 1.4e-6 + (reduce ? 3.3 : 0.0) : 0.0);
+    struct Tile {
+        int tt, tiles;
+        bool r16;
+        double chunk, fixed;
+    } tile[5];
+    int nt = 0;
+    auto add = [&](int tt, bool r16, double chunk, double fixed) {
+        if (only && ((std::strcmp(only, "r16") == 0) != r16 || (!r16 && std::atoi(only) != 16 * tt))) return;
+        tile[nt++] = Tile{tt, rt * ((n + 16 * tt - 1) / (16 * tt)), r16, unit * chunk, fixed};
+    };
+    add(2, false, 1.35, 2.2);
+    add(4, false, 1.65, 2.9);
+    add(6, false, 1.78, 4.5);
+    if (type != T_Q8_0) add(8, false, 1.9, 6.3);
+    if (!pair) add(4, true, n <= 64 ? 1.6 : 1.7, n <= 64 ? 1.2 : 2.7);  // (gemm_r_kernel takes one matrix)
+    GemmPlan best{2, 1, false};
+    double bt = 1e30;
+    const int smax = std::max(1, std::min(nchunk / 2, cap));
+    for (int cps = (nchunk + smax - 1) / smax; cps <= nchunk; cps++) {  // chunks per slice
+        const int s = (nchunk + cps - 1) / cps;
+        if ((nchunk + s - 1) / s != cps) continue;  // as many slices of fewer chunks
+        const double tail = s > 1 ? s * out * 1.4e-6 + (reduce ? 3.3 : 0.0) : 0.0;
+        for (int i = 0; i < nt; i++) {
+            const int wgs = tile[i].tiles * s, rest = wgs % 512;
+            const double per = tile[i].r16 ? wgs / 512 * 1.8 + (rest > 256 ? 1.8 : rest ? 1.0 : 0.0) : (wgs + 255) / 256;
+            const double t = per * (cps * tile[i].chunk + tile[i].fixed) + tail;
             if (t < bt) {
                 bt = t;
-                best = GemmPlan{tt, s};
+                best = GemmPlan{tile[i].tt, s, tile[i].r16};
             }
         }
     }
@@ -584,10 +826,17 @@ static GemmPlan gemm_plan(const DMat &m, int32_t n, size_t part_bytes) {
 
 int gemm_split(const DMat &m, int32_t n, size_t part_bytes) { return gemm_plan(m, n, part_bytes).split; }
 
-template <class G, int NP>
-static hipError_t gemm_launch_t(const GemmArgs &a, int blocks, int tt, hipStream_t st) {
+template <class G, class R, int NP>
+static hipError_t gemm_launch_t(const GemmArgs &a, int blocks, const GemmPlan &p, hipStream_t st) {
     const dim3 grid((unsigned)blocks), block(GM_THREADS);
-    switch (tt) {
+    if constexpr (NP == 1) {
+        if (p.r16) {
+            const dim3 one((unsigned)a.seg[0].nx, (unsigned)((a.n + 63) / 64), (unsigned)p.split);
+            hipLaunchKernelGGL((gemm_r_kernel<G, R>), a.nseg > 1 ? grid : one, block, 0, st, a);
+            return hipGetLastError();
+        }
+    }
+    switch (p.tt) {
     case 2: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 2>), grid, block, gm_lds<G>(2), st, a); break;
     case 4: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 4>), grid, block, gm_lds<G>(4), st, a); break;
     case 6: hipLaunchKernelGGL((gemm_q_kernel<G, NP, 6>), grid, block, gm_lds<G>(6), st, a); break;
@@ -599,11 +848,11 @@ static hipError_t gemm_launch_t(const GemmArgs &a, int blocks, int tt, hipStream
     return hipGetLastError();
 }
 template <int NP>
-static hipError_t gemm_launch(const GemmArgs &a, int blocks, int tt, hipStream_t st) {
+static hipError_t gemm_launch(const GemmArgs &a, int blocks, const GemmPlan &p, hipStream_t st) {
     switch (a.seg[0].m.type) {
-    case T_Q4_K: return gemm_launch_t<GQ4K, NP>(a, blocks, tt, st);
-    case T_Q6_K: return gemm_launch_t<GQ6K, NP>(a, blocks, tt, st);
-    default: return gemm_launch_t<GQ80, NP>(a, blocks, tt, st);
+    case T_Q4_K: return gemm_launch_t<GQ4K, RQ4K, NP>(a, blocks, p, st);
+    case T_Q6_K: return gemm_launch_t<GQ6K, RQ6K, NP>(a, blocks, p, st);
+    default: return gemm_launch_t<GQ80, RQ80, NP>(a, blocks, p, st);
     }
 }
 // appends one projection's blocks to the launch
@@ -625,12 +874,15 @@ hipError_t launch_gemm(const DMat &m, const uint16_t *x, int32_t n, float *c, fl
     a.n = n;
     int blocks = 0;
     gemm_seg(a, m, split > 1 ? part : c, p, GM_ROWS, blocks);
-    const hipError_t r = gemm_launch<1>(a, blocks, p.tt, st);
+    const hipError_t r = gemm_launch<1>(a, blocks, p, st);
     if (r != hipSuccess) return r;
     if (split > 1) {
         const int64_t total = (int64_t)n * m.rows;
         const int64_t nb = ((total + 3) / 4 + WG - 1) / WG;
-        hipLaunchKernelGGL(gemm_reduce, dim3((unsigned)nb), dim3(WG), 0, st, part, c, total, split);
+        // (the last group loads its last slice again: no more of them than the slices need)
+        if (split <= 2) hipLaunchKernelGGL(gemm_reduce<2>, dim3((unsigned)nb), dim3(WG), 0, st, part, c, total, split);
+        else if (split <= 4) hipLaunchKernelGGL(gemm_reduce<4>, dim3((unsigned)nb), dim3(WG), 0, st, part, c, total, split);
+        else hipLaunchKernelGGL(gemm_reduce<8>, dim3((unsigned)nb), dim3(WG), 0, st, part, c, total, split);
     }
     return hipGetLastError();
 }
@@ -651,10 +903,10 @@ hipError_t launch_gemm_swiglu(const DMat &gate, const DMat &up, const uint16_t *
     a.n = n;
     a.m2 = up;
     a.h = h;
-    const GemmPlan p = gemm_plan(gate.type, gemm_rt(gate, GM_ROWS / 2), gate.cols / GM_KC, n, 0.0, 1, false);
+    const GemmPlan p = gemm_plan(gate.type, gemm_rt(gate, GM_ROWS / 2), gate.cols / GM_KC, n, 0.0, 1, false, true);
     int blocks = 0;
     gemm_seg(a, gate, nullptr, p, GM_ROWS / 2, blocks);
-    return gemm_launch<2>(a, blocks, p.tt, st);
+    return gemm_launch<2>(a, blocks, p, st);
 }
 
 hipError_t launch_gemm_parts(const DMat &m, const uint16_t *x, int32_t n, float *part, size_t part_bytes, int *split,
@@ -689,7 +941,7 @@ hipError_t launch_gemm_parts_multi(const DMat *const *m, float *const *part, con
         split[i] = p.split;
         gemm_seg(a, *m[i], part[i], p, GM_ROWS, blocks);
     }
-    return gemm_launch<1>(a, blocks, p.tt, st);
+    return gemm_launch<1>(a, blocks, p, st);
 }
 
 }  // namespace oi

@@ -178,10 +178,10 @@ def test_gemm_workspace_split(kind, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 256), (127, 31, 256), (129, 33, 512), (130, 64, 768), (256, 65, 512),
                                    (40, 127, 1280), (132, 129, 256), (128, 200, 2304), (70, 300, 512)])
 def test_gemm_tile_edges(kind, m, n, k):
-    """One past and one short of the tiles (128 rows; 32, 64 and 128 tokens; chunks
-    of 256 in K halves; rows not a multiple of 4): f32 sums of exact products differ
-    from the float64 sum by at most K 2^-24 sum|w x|, and sum|w x| is about sqrt(K)
-    times the result's size for these random signs."""
+    """Small products with the tile that the plan gives them: rows on both sides of
+    128, tokens on both sides of 32 to 128, rows not a multiple of 4.  f32 sums of
+    exact products differ from the float64 sum by at most K 2^-24 sum|w x|, and
+    sum|w x| is about sqrt(K) times the result's size for these random signs."""
     rng = np.random.default_rng(m * 31 + n * 7 + k + kind)
     w = gemm_blocks(kind, m, k, rng)
     x = x16(rng.uniform(-1, 1, size=(n, k)))
@@ -192,9 +192,10 @@ def test_gemm_tile_edges(kind, m, n, k):
 @pytest.mark.parametrize("kind,m,n,k", [(8, 12288, 96, 4096), (8, 12289, 97, 1024), (8, 1537, 191, 256),
                                         (14, 4097, 192, 512), (12, 511, 95, 2048)])
 def test_gemm_96_token_tiles_and_odd_rows(kind, m, n, k):
-    """Sizes about multiples of 96 tokens, where that tile is chosen or just not, and
-    row counts whose results are stored a float per lane (not a multiple of 4);
-    the bound is test_gemm_tile_edges'.  The oracle takes the first and last tile's rows."""
+    """Larger products of tokens about multiples of 96 with the tile that the plan
+    gives them (96 tokens to the first), and row counts whose results are stored a
+    float per lane (not a multiple of 4); the bound is test_gemm_tile_edges'.  The
+    oracle takes the first and last tile's rows."""
     rng = np.random.default_rng(m + n + k + kind)
     w = gemm_blocks(kind, m, k, rng)
     x = x16(rng.uniform(-1, 1, size=(n, k)))
@@ -205,3 +206,21 @@ def test_gemm_96_token_tiles_and_odd_rows(kind, m, n, k):
         rows = part.shape[0]
         err = scaled_err(np.ascontiguousarray(y[:, r]), refcpu.gemm_f16(part.reshape(-1), kind, rows, k, x))
         assert err <= k ** 1.5 * 2.0 ** -24, "%d %dx%dx%d scaled error %.3g" % (kind, m, n, k, err)
+
+
+@pytest.mark.parametrize("kind", [12, 14, 8])
+@pytest.mark.parametrize("tile", ["32", "64", "96", "128", "r16"])
+@pytest.mark.parametrize("m,past,k", [(127, -1, 768), (129, 0, 512), (130, 1, 1280), (256, 3, 256), (260, 1, 4096)])
+def test_gemm_every_tile_at_its_edges(monkeypatch, kind, tile, m, past, k):
+    """Each kernel and token tile by itself, one token short of a tile, whole, and
+    past one, rows on both sides of a 128-row tile, K whole and in slices (4096
+    columns); the bound is test_gemm_tile_edges'."""
+    if (kind, tile) == (8, "128"):
+        pytest.skip("Q8_0 has no 128-token tile (its planes do not fit the LDS beside the activations)")
+    monkeypatch.setenv("OI_GEMM_TILE", tile)
+    n = (64 if tile == "r16" else int(tile)) + past
+    rng = np.random.default_rng(m * 31 + n * 7 + k + kind)
+    w = gemm_blocks(kind, m, k, rng)
+    x = x16(rng.uniform(-1, 1, size=(n, k)))
+    err = scaled_err(ggml.gemm(kind, w, m, k, x), refcpu.gemm_f16(w, kind, m, k, x))
+    assert err <= k ** 1.5 * 2.0 ** -24, "%d %s %dx%dx%d scaled error %.3g" % (kind, tile, m, n, k, err)

@@ -52,9 +52,9 @@ def test_prefill_logits_vs_oracle(make_model, name, n):
 
 
 def test_prefill_512_tokens_fused_gate_up(make_model):
-    """512 batched tokens on small-q4_k: 24 row tiles x 8 token tiles of the
-    gate/up GEMM need no K split, so the fused gate/up pass with the SwiGLU
-    epilogue runs (the 8B-shape prefill's path); logits and argmax vs the
+    """512 batched tokens on small-q4_k: 48 row tiles of 64 gate and 64 up rows and
+    4 tiles of 128 tokens fill half of the CUs, so the fused gate/up pass with the
+    SwiGLU epilogue runs (the 8B-shape prefill's path); logits and argmax vs the
     oracle."""
     path = make_model("small-q4_k")
     e, r = _engines(path, 1024)
@@ -87,6 +87,26 @@ def test_prefill_fused_gate_up_equals_unfused_at_8b_shape(make_model, monkeypatc
         finally:
             infer.engine_destroy(e)
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32)), scaled_err(out[0], out[1])
+
+
+@pytest.mark.parametrize("kind", [12, 14, 8])
+@pytest.mark.parametrize("tile", ["32", "64", "96", "128"])
+def test_prefill_fused_gate_up_of_every_type_and_tile(make_model, monkeypatch, kind, tile):
+    """296 tokens (the last tile of every size ragged) through each type's and tile's
+    fused gate/up pass: 48 row tiles of a 3072-row pair; logits vs the oracle."""
+    if (kind, tile) == (8, "128"):
+        pytest.skip("Q8_0 has no 128-token tile")
+    path = make_model("tiny-q8_0", hidden_dim=3072, n_layers=1) if kind == 8 else \
+        make_model("tiny-q4_k", hidden_dim=3072, n_layers=1, type_default=kind)
+    monkeypatch.setenv("OI_GEMM_TILE", tile)
+    e, r = _engines(path, 512)
+    try:
+        toks = _tokens(kind, 296, r.vocab_size)
+        err = scaled_err(infer.engine_forward_batch(e, toks, 0), r.prefill(toks, 0))
+        assert err <= TOL, "scaled error %.3g" % err
+    finally:
+        infer.engine_destroy(e)
+        r.close()
 
 
 def _greedy_ref(r, token, pos, n):
