@@ -94,7 +94,11 @@ const float *oi_engine_forward(oi_engine *e, int32_t token, int32_t pos);
  * batched: the seven projections of each layer on the matrix cores with f16
  * operands and f32 accumulation (the reference's MMQ), the per-token operations
  * (norms, RoPE, cache store, causal attention, SwiGLU, residuals) in f32; the
- * trailing 1-7 tokens in oi_engine_forward's f32 arithmetic.  A model whose
+ * trailing 1-7 tokens in oi_engine_forward's f32 arithmetic, 2-7 of them in one
+ * pass over the weights (3-7 on a model with routed experts or DeltaNet layers; one
+ * at a time where the gate and up projections differ in type).  That pass's sums are
+ * in another order: a row agrees with oi_engine_forward's to f32 rounding, not bit
+ * for bit.  A model whose
  * projections the batched kernels cannot take (type other than Q4_K / Q6_K /
  * Q8_0, or a row length not a multiple of 256) runs every token through that
  * path, as the reference's non-Metal fallback (qwen3_5/engine.odin:86-91).  NULL on
@@ -104,7 +108,8 @@ const float *oi_engine_prefill(oi_engine *e, const int32_t *tokens, int32_t n, i
 /* engine_verify_batch (qwen3_5/engine.odin:166-174: forward_gpu_batch, then
  * metal_verify_batch_logits, qwen3_5/metal.odin:1707-1747): consume
  * tokens[0..n) at positions pos0 .. pos0+n-1 exactly as oi_engine_prefill
- * does (same chunking, same state afterwards) and return the logits of every
+ * does (same chunking, same state afterwards, the last row its result bit for
+ * bit) and return the logits of every
  * position: n rows of vocab_size floats, row i predicting position pos0+i+1
  * (engine-owned pinned host memory, valid until the next call of this
  * procedure).  Each row is the final RMSNorm and classifier of that token's

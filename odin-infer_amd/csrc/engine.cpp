@@ -1412,8 +1412,9 @@ int prefill_moe(oi_engine *e, const LayerDev &L, int T, bool combine = true) {
 // logits to rows + t * vocab (engine_verify_batch); otherwise the last token's
 // logits to e->logits.
 // Projections of the same f16 input into partial-product buffers P[idx[i]]
-// (slice counts to split[i]): consecutive matrices of one type share a launch
-// (launch_gemm_parts_multi; the same blocks and results as a launch each).
+// (slice counts to split[i]): consecutive matrices of one type share a launch and its
+// plan (launch_gemm_parts_multi), so a matrix's K slices need not be those of a
+// launch of its own.
 int prefill_projections(oi_engine *e, const DMat *const *m, const int *idx, int n, int T, int *split) {
     for (int i = 0; i < n;) {
         int j = i + 1;
@@ -1431,8 +1432,8 @@ int prefill_projections(oi_engine *e, const DMat *const *m, const int *idx, int 
     return OI_OK;
 }
 
-// The final RMSNorm and classifier of pf_x rows [t0, t0 + n) in f32 (the token
-// step's arithmetic, each row's result the same in any group), row i's logits to
+// The final RMSNorm and classifier of pf_x rows [t0, t0 + n) in f32 (each row's
+// result the same in any group, and the token step's where gemv_nt_repeats), row i's logits to
 // out + i * vocab: up to GEMV_NT_MAX rows per pass over the classifier, which was
 // read once for every row (151936 x 4096 Q6_K: 79 us a row).
 static int prefill_classify(oi_engine *e, int t0, int n, float *out) {
@@ -1576,7 +1577,9 @@ int prefill_chunk(oi_engine *e, const int32_t *tokens, int T, int pos, float *ro
 // The trailing 2-7 tokens of a call in one pass over the layers, in the arithmetic
 // of the token step (f32 activations, nothing staged in half): its GEMVs for all
 // the tokens at once (launch_gemv_nt), f32 attention, DeltaNet (token by token) and
-// routed experts between them.  Each trailing token through the token
+// routed experts between them.  Its sums are in another order than the token step's
+// (long rows in passes, the keys in other ranges), so a row differs from the token
+// step's by f32 rounding.  Each trailing token through the token
 // step reads every weight again: five tokens of the 8B shape took 5 x 1.85 ms.
 int prefill_few(oi_engine *e, const int32_t *tokens, int T, int pos, float *rows) {
     const hipStream_t st = e->stream;
@@ -1669,7 +1672,7 @@ int prefill_few_min(const oi_engine *e) {
 }
 
 // engine_forward_batch over tokens[0, n) at pos0 (chunks of a multiple of 8
-// up to PF_MAX_T batched, the trailing 1-7 in the decode path's arithmetic).  rows ==
+// up to PF_MAX_T batched, the trailing 1-7 in the decode path's f32 arithmetic).  rows ==
 // nullptr: the last token's logits in e->logits; otherwise every token's
 // logits, token i at rows + i * vocab (device memory).  Returns 0 or a code.
 int prefill_run(oi_engine *e, const int32_t *tokens, int32_t n, int32_t pos0, float *rows) {

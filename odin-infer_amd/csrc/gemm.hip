@@ -14,12 +14,12 @@
 // accumulators (TT / 2 tiles of 32 tokens), so every weight is dequantized once
 // per workgroup; the two K halves are added through LDS at the end.
 //
-// What bounds it, per chunk and CU at TT = 8 (clocks): the products 2048 (128 x
-// 128 x 256), the LDS ~2900 at 128 bytes a clock (staging, and the activations read
-// by four row groups), the vector instructions ~1900 with the products' issue,
-// the loads ~1700; alone 1.57 us a chunk, and 2.1 - 2.2 with every CU busy on
-// random data, where the card lowers its clock (a plain 8192^3 f16 product: 1795
-// TFLOP/s on zeros, 1315 on random data).  Measured on the way:
+// What bounds it: no unit, but how far two waves a SIMD with two barriers a chunk
+// overlap them.  Per chunk at TT = 8 (counters, gate and up of the 8B shape at 512
+// tokens), of 4800 clocks: the products 2050 a SIMD, the vector instructions 2090 with
+// the products' issue, the LDS 2170 and 170 of conflicts; 1.57 us a chunk alone and
+// 2.1 - 2.3 with every CU busy on random data, where the card lowers its clock (a plain
+// 8192^3 f16 product: 1795 TFLOP/s on zeros, 1315 on random data).  Measured on the way:
 //   - The weights go through LDS because of the loads: straight into the operand
 //     layout (16 rows x 64 bytes per instruction, the row in the fast lanes) a
 //     16-byte-per-lane load takes 65 clocks of the CU's address unit, with the

@@ -1446,7 +1446,7 @@ __device__ __forceinline__ int block_excl_scan(int v, int *wsum, int *total) {
 // row tile) of the gate/up and down multi-token GEMVs: tiles_gu / tiles_dn
 // row tiles per slice of pair_slice pairs of each chosen expert.
 __global__ __launch_bounds__(1024) void pf_moe_group_kernel(PfMoeArgs a) {
-    __shared__ int cnt[1024], fill[1024], sl[1025], wsum[16];
+    __shared__ int cnt[1024], fill[1024], sl[1024], wsum[16];
     const bool shared = a.kp > a.top_k;  // slot top_k of every token is the shared expert, expert n_experts
     const int ne = a.n_experts + (shared ? 1 : 0), P = a.T * a.kp, e = threadIdx.x;
     if (e < ne) {
@@ -1483,7 +1483,6 @@ __global__ __launch_bounds__(1024) void pf_moe_group_kernel(PfMoeArgs a) {
     }
     sl[e] = os;
     if (e == 0) {
-        sl[1024] = ts;
         a.nitems[0] = ts * a.tiles_gu;
         a.nitems[1] = ts * a.tiles_dn;
     }

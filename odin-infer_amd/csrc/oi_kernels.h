@@ -217,7 +217,7 @@ struct GemvNtArgs {
     const float *x;
     const float *norm_w;         // if set: x is replaced by rmsnorm(x) * norm_w
     float eps;
-    // the plan (plan_gemv_nt): columns per pass, lanes per row, workgroups, rows of the largest workgroup
+    // launch_gemv_nt's plan: columns per pass, lanes per row, workgroups, rows of the largest workgroup
     int32_t ks, lpr, total_wgs, rows_wg;
 };
 // whether the kernel takes the matrices (one type and row length)
@@ -261,8 +261,8 @@ struct PfQkvArgs {
 hipError_t launch_pf_qkv(const PfQkvArgs &a, int head_dim, hipStream_t st);
 // gate: null, or [T][n_heads * head_dim] f32, the output multiplied by its
 // sigmoid before rounding (the Qwen3.5 attention's output gate)
-// ws: optional scratch for the key-split form of short chunks (head_dim 256:
-// [splits][T][n_heads][head_dim + 2] floats, splits <= 16); unused if too small
+// ws: optional scratch for splitting the keys of a query tile over workgroups
+// ([splits][T][n_heads][head_dim + 2] floats, splits <= 16); fewer or none if too small
 hipError_t launch_pf_attn(const float *q, const uint16_t *kc, const uint16_t *vc, uint16_t *out, int T, int pos0,
                           int seq_len, int n_heads, int n_kv_heads, int head_dim, hipStream_t st,
                           const float *gate = nullptr, float *ws = nullptr, size_t ws_bytes = 0);

@@ -95,7 +95,7 @@ def engine_forward(e, token, pos):
 
 def engine_forward_batch(e, tokens, pos_start):
     """qwen3_5/engine.odin:61-93: consume `tokens` from `pos_start` (batched
-    chunks of a multiple of 8, up to 512; the trailing 1-7 one at a time);
+    chunks of a multiple of 8, up to 512; the trailing 1-7 in f32);
     returns the last token's logits (a view of engine memory)."""
     t = np.ascontiguousarray(tokens, np.int32)
     p = _native.hip().oi_engine_prefill(e.handle, t.ctypes.data, int(t.size), int(pos_start))

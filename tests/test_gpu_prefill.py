@@ -2,7 +2,7 @@
 qwen3_5/engine.odin:61-93) against the CPU oracle's restatement of the same
 path (refcpu.ref_engine_prefill: chunks of a multiple of 8 up to 512 tokens
 with f16-staged projections summed exactly, the trailing 1-7 tokens per
-token).
+token, where the GPU takes 2-7 of them in one pass of the same arithmetic).
 
 Bars: last-token logits within a scaled error max|d|/max|ref| <= 1e-3 of the
 oracle and the same argmax; greedy continuation after the prefill identical to

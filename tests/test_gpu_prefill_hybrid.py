@@ -4,7 +4,7 @@ for the full-attention and DeltaNet layers; the routed-expert FFN, which the
 reference's batched path does not have, in f32 as the per-token path) against
 the oracle's restatement (refcpu.ref_engine_prefill: staged attention /
 DeltaNet / dense-MLP projections, the routed experts exact, the trailing 1-7
-tokens per token).
+tokens per token, where the GPU takes 3-7 of them in one pass).
 
 Bars: last-token logits within a scaled error of 1e-3 and the same argmax;
 the state the chunk leaves (K/V of the full-attention layers, conv and
@@ -426,8 +426,8 @@ def test_prefill_attention_kernels_agree(make_model, monkeypatch, n):
 @pytest.mark.parametrize("name,seed", [("tiny-q4_k", 31), ("moe-tiny", 43), ("qwen35-moe-tiny", 194)])
 def test_verify_batch_vs_oracle(make_model, name, seed):
     """engine_verify_batch (qwen3_5/engine.odin:166-174): after a 20-token
-    prompt, 11 draft tokens (a batched chunk of 8, then 3 through the token
-    path) with every position's logits returned.  Each row within 1e-3 of the
+    prompt, 11 draft tokens (a batched chunk of 8, then 3 in one f32
+    pass) with every position's logits returned.  Each row within 1e-3 of the
     oracle's verify_batch with the same argmax; the last row equals
     engine_forward_batch's result for the same tokens on a second engine, bit
     for bit (the same kernels); the state afterwards is the prefill's: the
