@@ -90,10 +90,12 @@ def test_prefill_fused_gate_up_equals_unfused_at_8b_shape(make_model, monkeypatc
 
 
 @pytest.mark.parametrize("kind", [12, 14, 8])
-@pytest.mark.parametrize("tile", ["32", "64", "96", "128"])
+@pytest.mark.parametrize("tile", ["32", "64", "96", "128", "r16"])
 def test_prefill_fused_gate_up_of_every_type_and_tile(make_model, monkeypatch, kind, tile):
     """296 tokens (the last tile of every size ragged) through each type's and tile's
-    fused gate/up pass: 48 row tiles of a 3072-row pair; logits vs the oracle."""
+    fused gate/up pass: 48 row tiles of a 3072-row pair; "r16", which takes one
+    matrix at a time, holds the other projections (q and k in one launch) to the
+    16-row-wave kernel; logits vs the oracle."""
     if (kind, tile) == (8, "128"):
         pytest.skip("Q8_0 has no 128-token tile")
     path = make_model("tiny-q8_0", hidden_dim=3072, n_layers=1) if kind == 8 else \

@@ -598,3 +598,18 @@ def test_last_verified_row_is_the_prefills(make_model, name, over, n):
     finally:
         infer.engine_destroy(e)
         infer.engine_destroy(s)
+
+
+@pytest.mark.parametrize("tile", ["32", "96", "r16"])
+def test_hybrid_projections_of_every_kernel(make_model, monkeypatch, tile):
+    """A hybrid's chunk of 136 tokens with its projections (the DeltaNet layers' four
+    in one launch) held to one tile or kernel; logits vs the oracle."""
+    path = make_model("qwen35-tiny")
+    monkeypatch.setenv("OI_GEMM_TILE", tile)
+    e, r = _engines(path, 256)
+    try:
+        toks = _tokens(61, 136, r.vocab_size)
+        assert scaled_err(infer.engine_forward_batch(e, toks, 0), r.prefill(toks, 0)) <= TOL
+    finally:
+        infer.engine_destroy(e)
+        r.close()
